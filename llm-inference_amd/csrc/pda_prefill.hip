@@ -39,6 +39,9 @@
 //    query heads that read one kv head's tile are dispatched back to back to
 //    one XCD (workgroups go round robin over the 8 XCDs), so the L2 of that
 //    XCD serves the tile to all of them.
+//  * 16-bit K/V at D <= 256 runs the pipelined form of this loop
+//    (prefill_pipe_body); 8-bit K/V, D = 512 and the generic head dims run
+//    the form described so far (prefill_body).
 //  * LDS rows are padded so that the 16 lanes of a 16-byte K read, and the
 //    four rows of a transposed V read, fall on distinct banks.
 //  * Other even head dims up to 512 (GEN) run the kernel of the next of
@@ -54,6 +57,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "pda.h"
 #include "pda_internal.h"
@@ -152,6 +156,114 @@ __device__ __forceinline__ f16 round16(float x) {
 // Keys per tile: 64 (two 32-key blocks) where the registers allow it.
 template <int D>
 constexpr int blocks_per_tile() { return D <= 128 ? 2 : 1; }
+
+// LDS byte address of a shared object.
+__device__ __forceinline__ uint32_t lds_address(const void* at) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)at;
+}
+
+// 16 bytes per lane from global memory straight into LDS: lane i's, from src +
+// kOff bytes, to dst + kOff + kPlus + 16 i (dst: wave-uniform; the
+// instruction adds its offset to both addresses). The caller waits
+// (wait_vmem0) before the barrier that publishes them.
+template <int kOff, int kPlus>
+__device__ __forceinline__ void copy_to_lds(const void* src, uint32_t dst) {
+  asm volatile("s_add_u32 m0, %0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%3" ::"s"(
+                   dst),
+               "v"(src), "n"(kPlus), "n"(kOff)
+               : "memory", "m0", "scc");
+}
+
+// The same product added to c; kAcc: c in accumulator registers, which the
+// compiler would otherwise copy to vector registers and back. (The compiler
+// does not know what such an instruction still has in flight: c is only read
+// by further ones until outputs_done; s_nop: operands a VALU instruction has
+// just written.)
+template <bool BF, bool kAcc>
+__device__ __forceinline__ void mfma_to(const f16x8& a, const f16x8& b, f32x16& c) {
+  if constexpr (!kAcc)
+    c = mfma16<BF>(a, b, c);
+  else if constexpr (BF)
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+// f(0), f(1), ... with compile-time arguments.
+template <class F, int... kI>
+__device__ __forceinline__ void each(F& f, std::integer_sequence<int, kI...>) {
+  (f(std::integral_constant<int, kI>{}), ...);
+}
+
+__device__ __forceinline__ void wait_vmem0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
+// Output of one query: normalised, or the unnormalised partial of a key range.
+template <int D, bool BF, bool GEN, bool ODD>
+__device__ __forceinline__ void finish(const PrefillParams& p,
+                                       const f32x16 (&o)[D / slices_for(D) / 32], float m, float l,
+                                       int qi, int h, int split, int hh, int sl, bool q_live) {
+  constexpr int kDW = D / slices_for(D);
+  if (!q_live) return;
+  l += __shfl_xor(l, 32);
+  if (p.splits > 1) {
+    // Unnormalised partial and its (max, sum) for the merge; an empty or
+    // fully masked range leaves m = -inf, l = 0 and zeros.
+    const int64_t at = ((int64_t)split * p.count + qi) * p.hq + h;  // partials are D wide
+    float* dst = p.part_o + at * D + sl * kDW;
+#pragma unroll
+    for (int b = 0; b < kDW / 32; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4*>(dst + 32 * b + 8 * g + 4 * hh) =
+            make_float4(o[b][4 * g], o[b][4 * g + 1], o[b][4 * g + 2], o[b][4 * g + 3]);
+    if (hh == 0 && sl == 0) p.part_ml[at] = make_float2(m, l);
+    return;
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  if constexpr (ODD) {
+    // Rows of an odd number of elements: one element per store.
+    const int hd = p.head_dim;
+    f16* dst = p.out + ((int64_t)qi * p.hq + h) * hd;
+#pragma unroll
+    for (int b = 0; b < kDW / 32; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int d = sl * kDW + 32 * b + 8 * (v / 4) + 4 * hh + v % 4;
+        if (d < hd) dst[d] = round16<BF>(o[b][v] * inv);
+      }
+    return;
+  }
+  if constexpr (GEN) {
+    // Rows of head_dim elements: element pairs, the real dims only.
+    const int hd = p.head_dim;
+    f16* dst = p.out + ((int64_t)qi * p.hq + h) * hd;
+#pragma unroll
+    for (int b = 0; b < kDW / 32; ++b) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = sl * kDW + 32 * b + 8 * g + 4 * hh;
+        const f16x2 y0 = {round16<BF>(o[b][4 * g] * inv), round16<BF>(o[b][4 * g + 1] * inv)};
+        const f16x2 y1 = {round16<BF>(o[b][4 * g + 2] * inv),
+                          round16<BF>(o[b][4 * g + 3] * inv)};
+        if (d < hd) *reinterpret_cast<f16x2*>(dst + d) = y0;
+        if (d + 2 < hd) *reinterpret_cast<f16x2*>(dst + d + 2) = y1;
+      }
+    }
+    return;
+  }
+  f16* dst = p.out + ((int64_t)qi * p.hq + h) * D + sl * kDW;
+  // O^T rows: element 32 b + 8 (v / 4) + 4 hh + v % 4 of query n (of the slice).
+#pragma unroll
+  for (int b = 0; b < kDW / 32; ++b) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f16x4 y;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) y[t] = round16<BF>(o[b][4 * g + t] * inv);
+      *reinterpret_cast<f16x4*>(dst + 32 * b + 8 * g + 4 * hh) = y;
+    }
+  }
+}
 
 // Q8: the arena holds int8 rows and fp16 scales; the gather dequantizes each
 // row to fp16(int8 x scale) on its way into LDS, the values the reference's
@@ -741,66 +853,551 @@ __device__ __forceinline__ void prefill_body(const PrefillParams p) {
     __syncthreads();  // the next tile is in LDS; this one may be overwritten
   }
 
-  if (!q_live) return;
-  l += __shfl_xor(l, 32);
-  if (p.splits > 1) {
-    // Unnormalised partial and its (max, sum) for the merge; an empty or
-    // fully masked range leaves m = -inf, l = 0 and zeros.
-    const int64_t at = ((int64_t)split * p.count + qi) * p.hq + h;  // partials are D wide
-    float* dst = p.part_o + at * D + sl * kDW;
-#pragma unroll
-    for (int b = 0; b < kDW / 32; ++b)
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<float4*>(dst + 32 * b + 8 * g + 4 * hh) =
-            make_float4(o[b][4 * g], o[b][4 * g + 1], o[b][4 * g + 2], o[b][4 * g + 3]);
-    if (hh == 0 && sl == 0) p.part_ml[at] = make_float2(m, l);
-    return;
+  finish<D, BF, GEN, ODD>(p, o, m, l, qi, h, split, hh, sl, q_live);
+}
+
+// ---------------------------------------------------------------------------
+// The pipelined kernels: 16-bit K/V at head dims 64, 96, 128 and 256.
+//
+// The tile loop of prefill_body computes S, softmax and P V of a tile one
+// after the other and moves K/V through registers on its way into LDS; a wave
+// spent 5,000 - 6,000 cycles on a 64-key tile at D = 128 that holds 1,024
+// cycles of matrix-core work, spread over every phase. Here
+//  * a step interleaves, instruction by instruction, the products of one
+//    32-key block's V, the scores of a later block and the weights of the
+//    block between them, so that one wave alone keeps the matrix core busy
+//    while its exps run (`step`);
+//  * K and V go from global memory straight into LDS (copies spread over the
+//    slots of a step: issued together they stalled a wave for 1,250 cycles a
+//    tile), in planes of 64 bytes per key whose reads touch each bank once:
+//    V as it lies, K with its 16-byte chunks permuted by key;
+//  * V runs one tile behind K, so that two LDS tiles of each serve the
+//    pipeline with one barrier per tile;
+//  * what only some tiles need (masks, softcap, the running max) sits behind
+//    one wave-uniform test per step.
+// What bounds it: at D = 128 with one query block a wave (two workgroups per
+// CU) a step takes 1,040 - 1,320 cycles for 1,024 of the two waves'
+// matrix-core work, and the power limit (2.0 GHz under this load, 2.3 GHz
+// with two blocks a wave, which read K and V from LDS half as often). 4096
+// tokens at 0, 28/4 heads: 158 -> 141 us; 512 at 32256: 279 -> 228 us; 4096 at
+// 32256 1.14 PFLOP/s. D = 64 (14/2 heads, 1531 at 389): 30.8 -> 26.0 us. D = 256
+// (16/8 heads, 2048 at 6144, window 1024): 80 -> 59 us.
+//
+// Measured and not kept: the weights' sum on v_dot2 inside the step (each
+// holds the matrix pipe for 18 cycles: step 1,156 against 1,040), fp32 adds
+// of the rounded weights instead (level), operands read 2, 4 or 5 ahead
+// instead of 3 (level), two query blocks a wave at D = 64 (31.7 us).
+//
+// QB: blocks of 32 queries per wave.
+template <int D, int QB, bool BF>
+__device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
+  constexpr int kKeys = 64;             // keys per tile: two 32-key blocks
+  constexpr int kPlanes = D / 32;       // 64-byte planes of a row
+  constexpr int kPlane = kKeys * 32;    // halves per plane of a tile
+  constexpr int kTile = kPlanes * kPlane;
+  // Outputs of 64 x 128 or 32 x 256 are 128 registers a lane: they live in
+  // the accumulator registers, one wave per SIMD.
+  constexpr bool kAcc = D * QB > 128;
+  __shared__ __align__(1024) f16 s_k[2][kTile];
+  __shared__ __align__(1024) f16 s_v[2][kTile];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = uniform(tid >> 6);
+  const int n = lane & 31;
+  const int hh = lane >> 5;
+
+  const int G = p.hq / p.hkv;
+  int item = blockIdx.x;
+  const int runs = p.tiles * p.splits * p.hkv;
+  const int full = runs / kXcds * kXcds;
+  if (item < full * G) {
+    int x = item % kXcds;
+    const int j = item / kXcds;
+    // Where the XCDs hold several query tiles at once (fewer than 8 kv
+    // heads), every other round hands them out in reverse, so that no XCD
+    // gets the longer tile each time.
+    if ((j / G) & 1 && kXcds % p.hkv == 0) x = kXcds - p.hkv - x / p.hkv * p.hkv + x % p.hkv;
+    item = ((j / G) * kXcds + x) * G + j % G;
   }
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  if constexpr (ODD) {
-    // Rows of an odd number of elements: one element per store.
-    const int hd = p.head_dim;
-    f16* dst = p.out + ((int64_t)qi * p.hq + h) * hd;
+  const int run = item / G;
+  const int h = (run % p.hkv) * G + (item - run * G);
+  const int kvh = run % p.hkv;
+  const int split = (run / p.hkv) % p.splits;
+  const int tile = p.tiles - 1 - run / p.hkv / p.splits;
+
+  // The wave's QB blocks of 32 queries; block j of a lane is query qi + 32 j.
+  const int q0 = tile * (128 * QB);
+  const int q1 = min(q0 + 128 * QB, p.count);
+  const int wq0 = q0 + 32 * QB * w;
+  const int qi = wq0 + n;
+  const int qpos = p.start + qi;
+  const bool wave_live = wq0 < p.count;
+  const int wfirst = p.start + wq0;
+  const int wlast = p.start + min(wq0 + 32 * QB - 1, p.count - 1);
+
+  f16x8 qf[QB][D / 16];
 #pragma unroll
-    for (int b = 0; b < kDW / 32; ++b)
+  for (int j = 0; j < QB; ++j) {
+    const bool live = qi + 32 * j < p.count;
+    const f16* qp = p.q + ((int64_t)(live ? qi + 32 * j : 0) * p.hq + h) * D + 8 * hh;
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c) {
+      const f16x8 x = *reinterpret_cast<const f16x8*>(qp + 16 * c);
+      qf[j][c] = live ? x : f16x8{};
+      // (Only ever matrix-core operands.)
+      if constexpr (kAcc) asm volatile("" : "+a"(qf[j][c]));
+    }
+  }
+
+  int last = p.start + q1 - 1;
+  int kfirst = p.window > 0 ? max(0, p.start + q0 - p.window + 1) : 0;
+  int img_lo[QB] = {}, img_hi[QB] = {}, wave_last = wlast;
+  bool wave_img = false;
+  for (int i = 0; i < p.num_images; ++i) {
+    const int a = p.images[2 * i], b = min(p.images[2 * i + 1], p.start + p.count);
+    if (a >= b) continue;
+#pragma unroll
+    for (int j = 0; j < QB; ++j)
+      if (qpos + 32 * j >= a && qpos + 32 * j < b) img_lo[j] = a, img_hi[j] = b;
+    if (a <= last && b > p.start + q0) {
+      last = max(last, b - 1);
+      kfirst = min(kfirst, a);
+    }
+    if (wave_live && a <= wlast && b > wfirst) {
+      wave_last = max(wave_last, b - 1);
+      wave_img = true;
+    }
+  }
+  const int kbase = kfirst / kKeys * kKeys;
+  const int ntile = (last - kbase) / kKeys + 1;
+  const int t_begin = (int)((int64_t)ntile * split / p.splits);
+  const int t_end = (int)((int64_t)ntile * (split + 1) / p.splits);
+  // Tiles [wa, wb) of the range that this wave's queries see.
+  int wa = t_begin, wb = wave_live ? min(t_end, (wave_last - kbase) / kKeys + 1) : t_begin;
+  if (p.window > 0 && !wave_img) wa = max(wa, (max(0, wfirst - p.window + 1) - kbase) / kKeys);
+  wa = uniform(wa);
+  wb = uniform(wb);
+
+  // Gather: thread tid moves key tid / 4 of a tile, 64-byte pieces.
+  const int gk = tid >> 2;
+  int kp = kbase + t_begin * kKeys + gk;
+  int pi = kp / p.page_size;
+  int r = kp - pi * p.page_size;
+  // 16-byte chunk of each 64-byte piece this lane fetches: K's are swizzled.
+  const int kchunk = 8 * ((lane & 3) ^ ((lane >> 4) & 3));
+  const int vchunk = 8 * (lane & 3);
+  const uint32_t k_dst = uniform(lds_address(&s_k[0][0]) + 1024 * w);
+  const uint32_t v_dst = uniform(lds_address(&s_v[0][0]) + 1024 * w);
+  // The page of this thread's key is looked up two iterations before its rows
+  // are copied, so nothing waits for it; each wave looks up the pages of all
+  // 64 keys of the tile as well (one per lane) for the mask of usable keys,
+  // which then needs neither LDS nor a barrier.
+  const uint32_t pages = (uint32_t)min(p.arena_pages, (int64_t)INT32_MAX);
+  const int step_pages = kKeys / p.page_size, step_rows = kKeys % p.page_size;
+  int page = 0, row_off = 0, page_m = 0;
+  bool in = false, in_m = false;
+  int kp_m = kbase + t_begin * kKeys + lane;
+  int pi_m = kp_m / p.page_size;
+  int r_m = kp_m - pi_m * p.page_size;
+  auto lookup = [&]() {
+    in = kp <= last && pi < p.table_len;
+    in_m = kp_m <= last && pi_m < p.table_len;
+    page = p.table[min(pi, p.table_len - 1)];
+    page_m = p.table[min(pi_m, p.table_len - 1)];
+    row_off = r * p.row_elems + kvh * p.head_elems;
+    kp += kKeys;
+    kp_m += kKeys;
+    r += step_rows;
+    r_m += step_rows;
+    pi += step_pages + (r >= p.page_size ? 1 : 0);
+    pi_m += step_pages + (r_m >= p.page_size ? 1 : 0);
+    r -= r >= p.page_size ? p.page_size : 0;
+    r_m -= r_m >= p.page_size ? p.page_size : 0;
+  };
+  // This thread's rows of the tiles whose V and K are copied next, their
+  // usable keys, and those of the tile after them.
+  const f16* src_k = nullptr;
+  const f16* src_v = nullptr;
+  uint64_t at_k = 0;
+  bool ok_k = false, ok_v = false;
+  uint64_t ok_prev = 0, ok_now = 0, ok_next = 0;
+  // Takes the looked-up tile as the next K to copy, the one before it as the
+  // next V.
+  auto advance = [&]() {
+    src_v = static_cast<const f16*>(p.v) + at_k + vchunk;
+    ok_v = ok_k;
+    ok_prev = ok_now;
+    ok_now = ok_next;
+    ok_k = in && (uint32_t)page < pages;
+    ok_next = __ballot(in_m && (uint32_t)page_m < pages);
+    at_k = (uint64_t)(uint32_t)(ok_k ? page : 0) * (uint32_t)p.page_elems + (uint32_t)row_off;
+    src_k = static_cast<const f16*>(p.k) + at_k + kchunk;
+  };
+  auto copy_k = [&](int buf, auto i) {
+    copy_to_lds<64 * i.value, (2 * kPlane - 64) * i.value>(src_k, k_dst + buf * (2 * kTile));
+  };
+  auto copy_v = [&](int buf, auto i) {
+    copy_to_lds<64 * i.value, (2 * kPlane - 64) * i.value>(src_v, v_dst + buf * (2 * kTile));
+  };
+  // After the copies have landed: rows of unusable keys become zeros (their
+  // weight is 0; zero V keeps 0 * V finite whatever the arena holds there).
+  auto clean_v = [&](int buf, bool ok) {
+    if (!ok) {
+#pragma unroll
+      for (int i = 0; i < kPlanes; ++i)
+        *reinterpret_cast<f16x8*>(&s_v[buf][kPlane * i + 32 * gk + 8 * (lane & 3)]) = f16x8{};
+    }
+  };
+
+  f32x16 o[QB][D / 32];
+  float m[QB], l[QB];
+#pragma unroll
+  for (int j = 0; j < QB; ++j) {
+    m[j] = -INFINITY;
+    l[j] = 0.0f;
+#pragma unroll
+    for (int b = 0; b < D / 32; ++b) o[j][b] = f32x16{};
+  }
+  f32x16 s0[QB] = {}, s1[QB] = {};  // scores of the even and the odd 32-key block
+  f16x8 p0[QB][2] = {}, p1[QB][2] = {};  // and their weights
+
+  const int g16 = lane >> 4, s16 = lane & 15;
+  const int v_lane = (4 * (g16 >> 1) + (s16 >> 2)) * 32 + 16 * (g16 & 1) + 4 * (s16 & 3);
+  const int ksw = (n >> 2) & 3;
+  const int k_lane0 = 32 * n + 8 * (hh ^ ksw);
+  const int k_lane1 = 32 * n + 8 * ((2 + hh) ^ ksw);
+  const float c = p.softcap <= 0.0f && p.scale_log2 > 0.0f ? p.scale_log2 : 1.0f;
+
+  // Bits 0 .. n - 1 (none for n <= 0, all from 32 on).
+  auto below = [](int n) -> uint32_t {
+    const uint32_t ones = n >= 32 ? 32u : n > 0 ? (uint32_t)n : 0u;
+    return (uint32_t)((1ull << ones) - 1);
+  };
+  // Scores of a block in place: softcap or a scale that is not positive,
+  // then the masks.
+  auto shape = [&](f32x16 (&xs)[QB], int k0, uint32_t okm) {
+#pragma unroll
+    for (int j = 0; j < QB; ++j) {
+      f32x16& x = xs[j];
+      if (p.softcap > 0.0f) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const float e = __builtin_amdgcn_exp2f(x[v] * p.cap_in);
+          x[v] = (1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f)) * p.cap_out;
+        }
+      } else if (!(p.scale_log2 > 0.0f)) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) x[v] = x[v] * p.scale_log2;
+      }
+      // Keys k0 .. k0 + 31 this lane's query sees, one bit each: usable, and
+      // not past its position, inside its window, or inside its image. Two
+      // instructions per score then (bit to mask, select), where a test of
+      // each key's position took nine: the diagonal tiles are most of a short
+      // prompt (4096 tokens: 12 of the 117 us of its longest workgroup).
+      const int hi = qpos + 32 * j - k0;
+      uint32_t see = below(hi + 1);
+      if (p.window > 0) see &= ~below(hi - p.window + 1);
+      if (wave_img) see |= below(img_hi[j] - k0) & ~below(img_lo[j] - k0);
+      see = (see & okm) >> (4 * hh);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int d = sl * kDW + 32 * b + 8 * (v / 4) + 4 * hh + v % 4;
-        if (d < hd) dst[d] = round16<BF>(o[b][v] * inv);
-      }
-    return;
-  }
-  if constexpr (GEN) {
-    // Rows of head_dim elements: element pairs, the real dims only.
-    const int hd = p.head_dim;
-    f16* dst = p.out + ((int64_t)qi * p.hq + h) * hd;
-#pragma unroll
-    for (int b = 0; b < kDW / 32; ++b) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = sl * kDW + 32 * b + 8 * g + 4 * hh;
-        const f16x2 y0 = {round16<BF>(o[b][4 * g] * inv), round16<BF>(o[b][4 * g + 1] * inv)};
-        const f16x2 y1 = {round16<BF>(o[b][4 * g + 2] * inv),
-                          round16<BF>(o[b][4 * g + 3] * inv)};
-        if (d < hd) *reinterpret_cast<f16x2*>(dst + d) = y0;
-        if (d + 2 < hd) *reinterpret_cast<f16x2*>(dst + d + 2) = y1;
+        const int bit = __builtin_amdgcn_sbfe((int)see, 8 * (v / 4) + (v % 4), 1);
+        const float y = x[v];  // (a bit cast of x[v] itself takes element 0)
+        x[v] = __builtin_bit_cast(float, (__builtin_bit_cast(int, y) & bit) |
+                                             (~bit & (int)0xFF800000));
       }
     }
-    return;
-  }
-  f16* dst = p.out + ((int64_t)qi * p.hq + h) * D + sl * kDW;
-  // O^T rows: element 32 b + 8 (v / 4) + 4 hh + v % 4 of query n (of the slice).
+  };
+  // Weights 2 i, 2 i + 1 of a block, rounded to 16 bits and packed.
+  auto put_pair = [&](f16x8 (&pb)[2], int i, float e0, float e1) {
+    f16x2 ph;
+    if constexpr (BF)
+      ph = __builtin_bit_cast(f16x2, bf16x2{(bf16)e0, (bf16)e1});
+    else
+      ph = f16x2{(f16)e0, (f16)e1};
+    pb[i / 4][2 * (i % 4)] = ph[0];
+    pb[i / 4][2 * (i % 4) + 1] = ph[1];
+  };
+  // Their sum, all of a block's at once: v_dot2 holds the matrix pipe, and
+  // one between two matrix-core instructions costs 18 cycles of it.
+  auto total = [&](const f16x8 (&pb)[2], float sum) {
+    float s2[2] = {sum, 0.0f};
 #pragma unroll
-  for (int b = 0; b < kDW / 32; ++b) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      f16x4 y;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) y[t] = round16<BF>(o[b][4 * g + t] * inv);
-      *reinterpret_cast<f16x4*>(dst + 32 * b + 8 * g + 4 * hh) = y;
+    for (int i = 0; i < 8; ++i) {
+      const f16x2 ph = {pb[i / 4][2 * (i % 4)], pb[i / 4][2 * (i % 4) + 1]};
+      if constexpr (BF)
+        s2[i & 1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, ph),
+                                                    bf16x2{(bf16)1.0f, (bf16)1.0f}, s2[i & 1], false);
+      else
+        s2[i & 1] = __builtin_amdgcn_fdot2(ph, f16x2{(f16)1.0f, (f16)1.0f}, s2[i & 1], false);
     }
+    return s2[0] + s2[1];
+  };
+  auto scores = [&](f32x16 (&x)[QB], const f16* kt) {
+#pragma unroll
+    for (int cc = 0; cc < D / 16; ++cc) {
+      const f16x8 a = *reinterpret_cast<const f16x8*>(kt + (cc & 1 ? k_lane1 : k_lane0) +
+                                                      kPlane * (cc >> 1));
+#pragma unroll
+      for (int j = 0; j < QB; ++j) x[j] = mfma16<BF>(a, qf[j][cc], cc == 0 ? f32x16{} : x[j]);
+    }
+  };
+  auto accumulate = [&](const f16x8 (&pb)[QB][2], const f16* vt) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int b = 0; b < D / 32; ++b) {
+        const f16* vp = vt + v_lane + kPlane * b + 512 * ks;
+        const f16x4 lo4 = read_tr(vp);
+        const f16x4 hi4 = read_tr(vp + 256);
+        const f16x8 a = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+#pragma unroll
+        for (int j = 0; j < QB; ++j) mfma_to<BF, kAcc>(a, pb[j][ks], o[j][b]);
+      }
+    }
+  };
+  // Before the outputs are read by anything but a matrix-core instruction.
+  auto outputs_done = [&]() {
+    if constexpr (kAcc) {
+      asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+      for (int j = 0; j < QB; ++j)
+#pragma unroll
+        for (int b = 0; b < D / 32; ++b) asm volatile("" : "+a"(o[j][b]));
+    }
+  };
+  // The weights of a block were taken against the running max and summed in
+  // lb. A weight past 2^8 (which keeps 16-bit weights finite) makes lb pass
+  // it; only then, or while no key was visible (lb then is infinite), the max
+  // is taken and the block weighed again.
+  auto settle = [&](const f32x16 (&xs)[QB], f16x8 (&pb)[QB][2], float (&lb)[QB]) {
+    bool again = false;
+#pragma unroll
+    for (int j = 0; j < QB; ++j) again |= !(lb[j] <= 256.0f);
+    if (__ballot(again) != 0) {
+      outputs_done();
+#pragma unroll
+      for (int j = 0; j < QB; ++j) {
+        const f32x16& x = xs[j];
+        float top = x[0];
+#pragma unroll
+        for (int v = 1; v < 16; ++v) top = fmaxf(top, x[v]);
+        top = fmaxf(top, __shfl_xor(top, 32)) * c;
+        if (top > m[j] + kSlack) {
+          const float f = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - top);
+          m[j] = top;
+          l[j] *= f;
+#pragma unroll
+          for (int b = 0; b < D / 32; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[j][b][v] *= f;
+        }
+        const float mu = m[j] == -INFINITY ? 0.0f : m[j];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          put_pair(pb[j], i, __builtin_amdgcn_exp2f(fmaf(x[2 * i], c, -mu)),
+                   __builtin_amdgcn_exp2f(fmaf(x[2 * i + 1], c, -mu)));
+        lb[j] = total(pb[j], 0.0f);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < QB; ++j) l[j] += lb[j];
+  };
+  // One step of the pipeline, QB x D / 8 matrix-core instructions in slots:
+  // the products of a 32-key block's V (weights pv) alternate with the scores
+  // of a later block (xn), and the weights of the block between them (x, into
+  // pb, summed into lb) are spread over the slots, done two slots early.
+  // Operands are read kAhead operands early.
+  auto step = [&](const f32x16 (&x)[QB], f16x8 (&pb)[QB][2], const f16x8 (&pv)[QB][2],
+                  f32x16 (&xn)[QB], float (&lb)[QB], const f16* kt, const f16* vt, auto beside) {
+    constexpr int kOps = D / 8;  // operands: V and K fragments in turn
+    constexpr int kSlots = QB * kOps;
+    constexpr int kAhead = QB > 1 ? 3 : 4;
+    constexpr int kScores = 16 * QB;
+    float mu[QB], e[kScores];
+#pragma unroll
+    for (int j = 0; j < QB; ++j) {
+      mu[j] = m[j] == -INFINITY ? 0.0f : m[j];
+      lb[j] = m[j] == -INFINITY ? INFINITY : 0.0f;
+    }
+    f16x8 a[kOps];
+    auto read = [&](int i) {
+      if (i & 1) {
+        const int cc = i >> 1;
+        a[i] = *reinterpret_cast<const f16x8*>(kt + (cc & 1 ? k_lane1 : k_lane0) +
+                                               kPlane * (cc >> 1));
+      } else {
+        const int b = (i >> 1) % (D / 32), ks = (i >> 1) / (D / 32);
+        const f16* vp = vt + v_lane + kPlane * b + 512 * ks;
+        const f16x4 lo4 = read_tr(vp);
+        const f16x4 hi4 = read_tr(vp + 256);
+        a[i] = f16x8{lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+      }
+    };
+    auto pair = [&](int i) {
+      put_pair(pb[i / 8], i % 8, e[2 * i], e[2 * i + 1]);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) read(i);
+    e[0] = fmaf(x[0][0], c, -mu[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    auto slot = [&](auto sc) {
+      constexpr int i = sc.value / QB, j = sc.value % QB;
+      if constexpr (i & 1) {
+        constexpr int cc = i >> 1;
+        xn[j] = mfma16<BF>(a[i], qf[j][cc], cc == 0 ? f32x16{} : xn[j]);
+      } else {
+        constexpr int b = (i >> 1) % (D / 32), ks = (i >> 1) / (D / 32);
+        mfma_to<BF, kAcc>(a[i], pv[j][ks], o[j][b]);
+      }
+      if constexpr (j == 0 && i + kAhead < kOps) read(i + kAhead);
+      if constexpr (j == QB - 1) beside(std::integral_constant<int, i>{});
+      constexpr int v0 = kScores * sc.value / (kSlots - 2);
+      constexpr int v1 = kScores * (sc.value + 1) / (kSlots - 2);
+#pragma unroll
+      for (int v = v0 < kScores ? v0 : kScores; v < (v1 < kScores ? v1 : kScores); ++v) {
+        // The argument of the next exp, this exp, the pair before.
+        if (v + 1 < kScores) e[v + 1] = fmaf(x[(v + 1) / 16][(v + 1) % 16], c, -mu[(v + 1) / 16]);
+        e[v] = __builtin_amdgcn_exp2f(e[v]);
+        if ((v & 1) && v >= 3) pair((v - 3) / 2);
+      }
+      if constexpr (sc.value == kSlots - 2) pair(kScores / 2 - 1);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    each(slot, std::make_integer_sequence<int, kSlots>{});
+#pragma unroll
+    for (int j = 0; j < QB; ++j) lb[j] = total(pb[j], lb[j]);
+    // Keeps the products of the step in it (they would sink past the branch
+    // of settle, away from the weights they are to overlap).
+#pragma unroll
+    for (int j = 0; j < QB; ++j) {
+      asm volatile("" : "+v"(xn[j]), "+v"(pb[j][0]), "+v"(pb[j][1]), "+v"(lb[j]));
+#pragma unroll
+      for (int b = 0; b < (kAcc ? 0 : D / 32); ++b) asm volatile("" : "+v"(o[j][b]));
+    }
+  };
+
+  // Whether the blocks of an iteration (the odd one of the tile before and
+  // the even one of this tile) need their masks, a softcap or an unusual scale.
+  const bool special = p.softcap > 0.0f || !(p.scale_log2 > 0.0f);
+  const int plain_hi = special ? INT32_MIN : wfirst - 31;
+  const int plain_lo = p.window > 0 ? wlast - p.window + 32 : INT32_MIN;
+  auto rough = [&](int k0) {
+    return k0 > plain_hi || k0 <= plain_lo || ((ok_prev >> 32) & (uint32_t)ok_now) != 0xFFFFFFFFu;
+  };
+  // Iteration t of the workgroup: V of tile t and K of tile t + 1 are copied
+  // beside the iteration's math and published by its barrier (close). The
+  // looked-up rows move on (turn) once the copies are issued.
+  auto each_plane = [&](auto f) { each(f, std::make_integer_sequence<int, kPlanes>{}); };
+  auto turn = [&]() {
+    advance();
+    lookup();
+  };
+  auto copies = [&](int t) {
+    const int buf = (t - t_begin) & 1;
+    each_plane([&](auto i) { copy_v(buf, i); });
+    each_plane([&](auto i) { copy_k(buf ^ 1, i); });
+  };
+  auto close = [&](int t, bool ok) {
+    wait_vmem0();
+    clean_v((t - t_begin) & 1, ok);
+    __syncthreads();
+  };
+  int t = t_begin;
+  lookup();
+  advance();
+  lookup();
+  each_plane([&](auto i) { copy_k(0, i); });
+  advance();
+  lookup();
+  wait_vmem0();
+  __syncthreads();
+  if (wa >= wb) wa = t_end;
+  auto idle = [&]() {  // an iteration whose tile this wave's queries do not see
+    const bool ok = ok_v;
+    copies(t);
+    turn();
+    close(t, ok);
+  };
+  for (; t < wa; ++t) idle();
+  float lb[QB];
+  auto unweighed = [&]() {
+#pragma unroll
+    for (int j = 0; j < QB; ++j) lb[j] = INFINITY;
+  };
+  if (t < t_end) {
+    // First tile: scores of both blocks, weights of the first.
+    {
+      const bool ok = ok_v;
+      copies(t);
+      const f16* kt = s_k[(t - t_begin) & 1];
+      const int k0 = kbase + t * kKeys;
+      scores(s0, kt);
+      shape(s0, k0, (uint32_t)ok_now);
+      scores(s1, kt + 1024);
+      unweighed();
+      settle(s0, p0, lb);
+      turn();
+      close(t, ok);
+    }
+    // Scores of tile t, weights of its even block and of tile t - 1's odd
+    // one, products of tile t - 1's V.
+    for (++t; t < wb; ++t) {
+      const int buf = (t - t_begin) & 1;
+      const int k0 = kbase + t * kKeys;
+      const f16* kt = s_k[buf];
+      const f16* vt = s_v[buf ^ 1];
+      const bool masks = rough(k0), ok = ok_v;
+      const uint32_t ok_even = (uint32_t)ok_now;
+      if (masks) shape(s1, k0 - 32, (uint32_t)(ok_prev >> 32));
+      step(s1, p1, p0, s0, lb, kt, vt, [&](auto i) {
+        if constexpr (i.value % 2 == 0) {
+          constexpr int j = i.value / 2;
+          if constexpr (j < kPlanes)
+            copy_v(buf, std::integral_constant<int, j>{});
+          else
+            copy_k(buf ^ 1, std::integral_constant<int, j - kPlanes>{});
+        }
+      });
+      settle(s1, p1, lb);
+      if (masks) shape(s0, k0, ok_even);
+      step(s0, p0, p1, s1, lb, kt + 1024, vt + 1024, [&](auto i) {
+        if constexpr (i.value == 1) turn();
+      });
+      settle(s0, p0, lb);
+      close(t, ok);
+    }
+    // Past the last tile: weights of its odd block, products of its V.
+    {
+      const bool ok = ok_v;
+      const uint32_t ok_odd = (uint32_t)(ok_prev >> 32);
+      if (t < t_end) copies(t);
+      const f16* vt = s_v[((t - t_begin) & 1) ^ 1];
+      shape(s1, kbase + t * kKeys - 32, ok_odd);
+      accumulate(p0, vt);
+      unweighed();
+      settle(s1, p1, lb);
+      accumulate(p1, vt + 1024);
+      if (t < t_end) {
+        turn();
+        close(t, ok);
+      }
+    }
+    for (++t; t < t_end; ++t) idle();
   }
+  outputs_done();
+#pragma unroll
+  for (int j = 0; j < QB; ++j)
+    finish<D, BF, false, false>(p, o[j], m[j], l[j], qi + 32 * j, h, split, hh, 0,
+                                qi + 32 * j < p.count);
+}
+
+template <int D, int QB, bool BF>
+__global__ __launch_bounds__(256, D * QB <= 128 ? 2 : 1) void paged_prefill_pipe_kernel(
+    const PrefillParams p) {
+  prefill_pipe_body<D, QB, BF>(p);
 }
 
 // The prefill kernel of every even head dim (template arguments as
@@ -869,34 +1466,6 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restr
 constexpr int kCus = 256;       // MI355X compute units
 constexpr int kMaxSplits = 64;
 
-// Key ranges per (query tile, head): 1 when the tiles and heads alone give
-// every workgroup slot of the GPU (CUs x the kernel's occupancy) its work,
-// else as many as fit the slots in one round: the ranges of a chunk over a
-// long prefix are all alike, so a partly filled second round would cost a
-// whole range's time. One exception: a causal chunk that fills at most one
-// round and whose first query tile sees at most half the keys of its last
-// (a prompt from position 0) takes 2 ranges, so that the halves of its
-// longest tiles run beside its short ones. Each range holds at least 8 key
-// tiles. `request` > 0 forces a count.
-int prefill_splits(int start, int count, int q_heads, int head_dim, int window, int request) {
-  if (request > 0) return request < kMaxSplits ? request : kMaxSplits;
-  const int queries = queries_for(head_dim);
-  const int64_t wgs = (int64_t)(count + queries - 1) / queries * q_heads;
-  const int occupancy = head_dim == 64 ? 3 : head_dim <= 128 ? 2 : 1;
-  const int64_t slots = (int64_t)kCus * occupancy;
-  const int keys = 32 * (head_dim <= 128 ? 2 : 1);
-  // Keys seen by the chunk's first and last query tiles.
-  const int64_t cap = window > 0 ? (int64_t)window + queries : INT64_MAX;
-  const int64_t first = std::min<int64_t>((int64_t)start + std::min(count, queries), cap);
-  const int64_t span = std::min<int64_t>((int64_t)start + count, cap);
-  const int64_t by_keys = (span + keys - 1) / keys / 8;
-  if (wgs * 2 > slots) return wgs <= slots && 2 * first <= span && by_keys >= 2 ? 2 : 1;
-  int64_t s = slots / wgs;
-  if (s > by_keys) s = by_keys;
-  if (s > kMaxSplits) s = kMaxSplits;
-  return s < 1 ? 1 : (int)s;
-}
-
 size_t prefill_workspace(int splits, int count, int q_heads, int head_dim) {
   if (splits <= 1) return 0;
   const size_t pairs = (size_t)count * q_heads;
@@ -920,7 +1489,11 @@ int prefill_dim(int head_dim) {
 
 template <bool Q8, bool BF, bool GEN>
 const void* prefill_kernel_for(int kdim) {
-  return kdim == 64    ? reinterpret_cast<const void*>(paged_prefill_kernel<64, Q8, BF, GEN>)
+  // 16-bit K/V at the narrower tuned head dims runs the pipelined kernels.
+  if constexpr (!Q8 && !GEN)
+    return reinterpret_cast<const void*>(paged_prefill_kernel<512, Q8, BF, GEN>);
+  else
+    return kdim == 64    ? reinterpret_cast<const void*>(paged_prefill_kernel<64, Q8, BF, GEN>)
          : kdim == 96  ? reinterpret_cast<const void*>(paged_prefill_kernel<96, Q8, BF, GEN>)
          : kdim == 128 ? reinterpret_cast<const void*>(paged_prefill_kernel<128, Q8, BF, GEN>)
          : kdim == 256 ? reinterpret_cast<const void*>(paged_prefill_kernel<256, Q8, BF, GEN>)
@@ -934,6 +1507,73 @@ const void* prefill_odd_kernel_for(int kdim) {
          : kdim == 128 ? reinterpret_cast<const void*>(paged_prefill_odd_kernel<128, Q8, BF>)
          : kdim == 256 ? reinterpret_cast<const void*>(paged_prefill_odd_kernel<256, Q8, BF>)
                        : reinterpret_cast<const void*>(paged_prefill_odd_kernel<512, Q8, BF>);
+}
+
+// How a call's work is cut.
+struct Shape {
+  bool pipe;      // the pipelined kernels
+  int blocks;     // query blocks per wave (pipelined)
+  int queries;    // per workgroup
+  int keys;       // per tile, as ranges are planned
+  int occupancy;  // workgroups per CU
+};
+
+// The pipelined kernels serve 16-bit K/V at head dims 64, 96, 128 and 256.
+// At 128 a wave may hold two blocks of queries (one wave per SIMD, half the
+// LDS reads per product): faster where the prefix is long (512 queries at
+// 32256: 228 us against 247; 4096 at 32256: 1771 against 1997), slower where
+// the chunk is short or the tiles few (512 at 0: 25 against 15 us; 1024 at
+// 4096 and 4096 at 0 level). The line is 8192 keys, and no workgroup of 256
+// queries may stay half empty (384 at 32256: 211 against 185 us).
+Shape shape_for(int head_dim, int kdim, bool q8, int start, int count, int window) {
+  const bool pipe =
+      !q8 && (head_dim == 64 || head_dim == 96 || head_dim == 128 || head_dim == 256);
+  if (!pipe)
+    return Shape{false, 1, queries_for(kdim), kdim <= 128 ? 64 : 32,
+                 kdim == 64 ? 3 : kdim <= 128 ? 2 : 1};
+  const int64_t keys = std::min<int64_t>((int64_t)start + count,
+                                         window > 0 ? (int64_t)window + count : INT64_MAX);
+  const int64_t tiles = ((int64_t)count + 127) / 128;
+  if (head_dim == 128 && keys >= 8192 && (tiles % 2 == 0 || tiles >= 8))
+    return Shape{true, 2, 256, 64, 1};
+  // (keys: the unit in which key ranges are planned, as for the other kernels.)
+  return Shape{true, 1, 128, head_dim == 256 ? 32 : 64, head_dim == 64 ? 3 : head_dim == 256 ? 1 : 2};
+}
+
+// Key ranges per (query tile, head): 1 when the tiles and heads alone give
+// every workgroup slot of the GPU (CUs x the kernel's occupancy) its work,
+// else as many as fit the slots in one round: the ranges of a chunk over a
+// long prefix are all alike, so a partly filled second round would cost a
+// whole range's time. One exception: a causal chunk that fills at most one
+// round and whose first query tile sees at most half the keys of its last
+// (a prompt from position 0) takes 2 ranges, so that the halves of its
+// longest tiles run beside its short ones. Each range holds at least 8 key
+// tiles. `request` > 0 forces a count.
+int prefill_splits(int start, int count, int q_heads, const Shape& sh, int window, int request) {
+  if (request > 0) return request < kMaxSplits ? request : kMaxSplits;
+  const int queries = sh.queries;
+  const int64_t wgs = (int64_t)(count + queries - 1) / queries * q_heads;
+  const int64_t slots = (int64_t)kCus * sh.occupancy;
+  const int keys = sh.keys;
+  // Keys seen by the chunk's first and last query tiles.
+  const int64_t cap = window > 0 ? (int64_t)window + queries : INT64_MAX;
+  const int64_t first = std::min<int64_t>((int64_t)start + std::min(count, queries), cap);
+  const int64_t span = std::min<int64_t>((int64_t)start + count, cap);
+  const int64_t by_keys = (span + keys - 1) / keys / 8;
+  if (wgs * 2 > slots) return wgs <= slots && 2 * first <= span && by_keys >= 2 ? 2 : 1;
+  int64_t s = slots / wgs;
+  if (s > by_keys) s = by_keys;
+  if (s > kMaxSplits) s = kMaxSplits;
+  return s < 1 ? 1 : (int)s;
+}
+
+template <bool BF>
+const void* pipe_kernel_for(int kdim, int blocks) {
+  return kdim == 64   ? reinterpret_cast<const void*>(paged_prefill_pipe_kernel<64, 1, BF>)
+         : kdim == 96 ? reinterpret_cast<const void*>(paged_prefill_pipe_kernel<96, 1, BF>)
+         : kdim == 256 ? reinterpret_cast<const void*>(paged_prefill_pipe_kernel<256, 1, BF>)
+         : blocks == 2 ? reinterpret_cast<const void*>(paged_prefill_pipe_kernel<128, 2, BF>)
+                       : reinterpret_cast<const void*>(paged_prefill_pipe_kernel<128, 1, BF>);
 }
 
 template <bool Q8, bool BF>
@@ -1003,9 +1643,12 @@ int prefill(const void* queries, const void* keys, const void* values, const voi
   if (q8 && (((uintptr_t)key_scales | (uintptr_t)value_scales) & 1))
     return fail(PDA_ERR_ALIGNMENT, "fp16 scale arenas must be 2-byte aligned");
   if ((uintptr_t)table & 3) return fail(PDA_ERR_ALIGNMENT, "the table must be 4-byte aligned");
-  const int nsplit = prefill_splits(start, count, q_heads, kdim, window, splits);
-  const int per_wg = queries_for(kdim);
-  if ((int64_t)((count + per_wg - 1) / per_wg) * q_heads * nsplit > INT32_MAX)
+  const Shape sh = shape_for(head_dim, kdim, q8, start, count, window);
+  const int nsplit = prefill_splits(start, count, q_heads, sh, window, splits);
+  const int per_wg = sh.queries;
+  // (Counted in the narrowest workgroups, whichever run.)
+  const int narrow = queries_for(kdim);
+  if ((int64_t)((count + (int64_t)narrow - 1) / narrow) * q_heads * nsplit > INT32_MAX)
     return fail(PDA_ERR_INVALID_ARGUMENT, "query tiles x query heads x splits exceeds 2^31");
   const size_t need = prefill_workspace(nsplit, count, q_heads, kdim);
   if (need > 0 && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)))
@@ -1048,7 +1691,7 @@ int prefill(const void* queries, const void* keys, const void* values, const voi
   prm.count = count;
   prm.tiles = (count + per_wg - 1) / per_wg;
   prm.splits = nsplit;
-  const int tile_keys = kdim <= 128 ? 64 : 32;
+  const int tile_keys = sh.keys;
   prm.page_step = tile_keys % page_size == 0 ? tile_keys / page_size : 0;
   prm.hq = q_heads;
   prm.hkv = kv_heads;
@@ -1060,12 +1703,13 @@ int prefill(const void* queries, const void* keys, const void* values, const voi
   prm.cap_in = softcap > 0.0f ? 2.0f * kLog2e * scale / softcap : 0.0f;
   prm.cap_out = softcap * kLog2e;
   void* args[] = {&prm};
-  const void* fn = q8 ? prefill_kernel_for<true, false>(kdim, gen, odd)
+  const void* fn = sh.pipe ? (bf16_elems ? pipe_kernel_for<true>(kdim, sh.blocks) : pipe_kernel_for<false>(kdim, sh.blocks))
+                  : q8 ? prefill_kernel_for<true, false>(kdim, gen, odd)
                   : bf16_elems ? prefill_kernel_for<false, true>(kdim, gen, odd)
                                : prefill_kernel_for<false, false>(kdim, gen, odd);
   const hipStream_t hs = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)((int64_t)prm.tiles * q_heads * nsplit));
-  hipError_t err = hipLaunchKernel(fn, grid, dim3(64 * waves_for(kdim)), args, 0, hs);
+  hipError_t err = hipLaunchKernel(fn, grid, dim3(sh.pipe ? 256 : 64 * waves_for(kdim)), args, 0, hs);
   if (err != hipSuccess)
     return fail(PDA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
   if (nsplit > 1) {
@@ -1100,9 +1744,14 @@ int pda_prefill_workspace_bytes(int32_t start, int32_t count, int32_t q_heads,
   const int kdim = prefill_dim(head_dim);
   if (kdim == 0)
     return fail(PDA_ERR_HEAD_DIM, "head_dim %d: prefill serves head dims 1..512", head_dim);
-  const int s = count == 0 ? 1 : prefill_splits(start, count, q_heads, kdim, window, splits);
+  // The same bytes for 16-bit and 8-bit caches, whose kernels differ.
+  int s = 1;
+  *bytes = 0;
+  for (int q8 = 1; q8 >= 0 && count > 0; --q8) {
+    s = prefill_splits(start, count, q_heads, shape_for(head_dim, kdim, q8, start, count, window), window, splits);
+    *bytes = std::max(*bytes, prefill_workspace(s, count, q_heads, kdim));
+  }
   if (splits_used) *splits_used = s;
-  *bytes = prefill_workspace(s, count, q_heads, kdim);
   return ok();
 }
 
