@@ -418,6 +418,35 @@ int pda_rope_append_q8(const void* q, void* q_out, const void* k, const void* v,
                        int64_t arena_rows, int32_t layout, int32_t rope_dims,
                        const float* inv_freq, void* stream);
 
+/* One layer's buffers of pda_rope_append_layers, with the meanings they have
+ * in pda_rope_append (scales: 8-bit arenas only, else NULL). */
+typedef struct pda_append_layer {
+  const void* q; /* all layers or none */
+  void* q_out;
+  const void* k;
+  const void* v;
+  void* k_arena;
+  void* v_arena;
+  void* key_scales;
+  void* value_scales;
+  int64_t arena_rows;
+} pda_append_layer;
+
+/* pda_rope_append (kv_bits 16; bf16_elems != 0: pda_rope_append_bf16) or
+ * pda_rope_append_q8 (kv_bits 8) for every layer of a step at once, for
+ * callers that have all layers' q, k and v before the first layer's
+ * attention (a captured step). Layers share everything but their buffers;
+ * what one layer writes must overlap nothing another layer reads or writes.
+ * `layers` is a host array, read before the call returns. Same bits as one
+ * call per layer. */
+int pda_rope_append_layers(const pda_append_layer* layers, int32_t num_layers,
+                           int32_t kv_bits, int32_t bf16_elems,
+                           const int32_t* positions, const int32_t* rows,
+                           int32_t n, int32_t q_heads, int32_t kv_heads,
+                           int32_t head_dim, int32_t page_size, int32_t layout,
+                           int32_t rope_dims, const float* inv_freq,
+                           void* stream);
+
 /* Device-side packing of one decode step's page tables. Replaces the host
  * packing of DecodeBatch.__init__ (batches.py:148-179: tables [B, width] int32
  * with 0 padding, lengths = positions + 1, write rows table[pos / P] * P +

@@ -108,7 +108,7 @@ __device__ __forceinline__ void rotate_head(const E* src, E* dst, float pos,
 // query heads first, then kv heads. No LDS and no barrier: every wave
 // computes the angles it uses (sincosf with full range reduction).
 template <typename E>
-__global__ __launch_bounds__(kAppendThreads) void rope_append_kernel(const AppendParams p) {
+__device__ __forceinline__ void append_body(const AppendParams& p) {
   const int t = blockIdx.x;
   const int lane = threadIdx.x & 63;
   const int h = blockIdx.y * kHeadsPerGroup + (threadIdx.x >> 6);
@@ -174,7 +174,7 @@ __device__ __forceinline__ void quantize_row(const f16 (&x)[kMaxPerLane], int d,
 
 // 8-bit K/V: as rope_append_kernel, with the rotated keys and the values
 // quantized per (row, kv head) into int8 arenas and fp16 scale arenas.
-__global__ __launch_bounds__(kAppendThreads) void rope_append_q8_kernel(const AppendParams p) {
+__device__ __forceinline__ void append_q8_body(const AppendParams& p) {
   const int t = blockIdx.x;
   const int lane = threadIdx.x & 63;
   const int h = blockIdx.y * kHeadsPerGroup + (threadIdx.x >> 6);
@@ -202,14 +202,61 @@ __global__ __launch_bounds__(kAppendThreads) void rope_append_q8_kernel(const Ap
   quantize_row(xv, p.d, lane, static_cast<int8_t*>(p.v_arena) + at, p.v_scale + sat);
 }
 
+template <typename E>
+__global__ __launch_bounds__(kAppendThreads) void rope_append_kernel(const AppendParams p) {
+  append_body<E>(p);
+}
+
+__global__ __launch_bounds__(kAppendThreads) void rope_append_q8_kernel(const AppendParams p) {
+  append_q8_body(p);
+}
+
+// Layers per launch: their pointers travel in the kernel arguments (72 bytes
+// a layer, of the 4 KB a launch may carry), so no device copy of them has to
+// live as long as a captured graph.
+constexpr int kMaxLayers = 48;
+
+struct AppendLayersParams {
+  AppendParams common;  // the per-layer fields are replaced by a layer's own
+  pda_append_layer layers[kMaxLayers];
+};
+static_assert(sizeof(AppendLayersParams) <= 4096, "kernel arguments");
+
+// One launch over layers: layer blockIdx.z, workgroups within it as in the
+// one-layer kernels. Latency bound like those. A captured step of 24 layers,
+// batch 8, 14/2 heads of 64, 1024 tokens: 408 us with an append before each
+// layer's attention, 340 us with this one launch.
+template <typename E, bool Q8>
+__global__ __launch_bounds__(kAppendThreads) void rope_append_layers_kernel(
+    const AppendLayersParams a) {
+  const pda_append_layer& l = a.layers[blockIdx.z];
+  AppendParams p = a.common;
+  p.q = static_cast<const f16*>(l.q);
+  p.q_out = static_cast<f16*>(l.q_out);
+  p.k = static_cast<const f16*>(l.k);
+  p.v = static_cast<const f16*>(l.v);
+  p.k_arena = l.k_arena;
+  p.v_arena = l.v_arena;
+  p.k_scale = static_cast<f16*>(l.key_scales);
+  p.v_scale = static_cast<f16*>(l.value_scales);
+  p.arena_rows = l.arena_rows;
+  if constexpr (Q8)
+    append_q8_body(p);
+  else
+    append_body<E>(p);
+}
+
 using pda_internal::fail;
 using pda_internal::ok;
 
-int rope_append(const void* q, void* q_out, const void* k, const void* v, void* k_arena,
-                void* v_arena, void* k_scale, void* v_scale, bool q8, bool bf16_elems,
-                const int32_t* positions, const int32_t* rows, int32_t n, int32_t q_heads,
-                int32_t kv_heads, int32_t head_dim, int32_t page_size, int64_t arena_rows,
-                int32_t layout, int32_t rope_dims, const float* inv_freq, void* stream) {
+// Checks one layer's call and fills in its parameters; prm.hq + prm.hkv is 0
+// where there is nothing to do.
+int append_params(const void* q, void* q_out, const void* k, const void* v, void* k_arena,
+                  void* v_arena, void* k_scale, void* v_scale, bool q8, const int32_t* positions,
+                  const int32_t* rows, int32_t n, int32_t q_heads, int32_t kv_heads,
+                  int32_t head_dim, int32_t page_size, int64_t arena_rows, int32_t layout,
+                  int32_t rope_dims, const float* inv_freq, AppendParams& prm) {
+  prm.hq = prm.hkv = 0;
   if (n < 0 || head_dim <= 0 || head_dim > kMaxHeadDim)
     return fail(PDA_ERR_INVALID_ARGUMENT, "n=%d head_dim=%d (need n >= 0, 0 < head_dim <= %d)",
                 n, head_dim, kMaxHeadDim);
@@ -247,7 +294,6 @@ int rope_append(const void* q, void* q_out, const void* k, const void* v, void* 
   if ((int64_t)hq + hkv > 65535LL * kHeadsPerGroup)
     return fail(PDA_ERR_INVALID_ARGUMENT, "too many heads (%d)", hq + hkv);
 
-  AppendParams prm;
   prm.q = static_cast<const f16*>(q);
   prm.q_out = static_cast<f16*>(q_out);
   prm.k = static_cast<const f16*>(k);
@@ -266,8 +312,22 @@ int rope_append(const void* q, void* q_out, const void* k, const void* v, void* 
   prm.half = rope_dims / 2;
   prm.page_size = page_size;
   prm.layout = layout;
+  return ok();
+}
+
+int rope_append(const void* q, void* q_out, const void* k, const void* v, void* k_arena,
+                void* v_arena, void* k_scale, void* v_scale, bool q8, bool bf16_elems,
+                const int32_t* positions, const int32_t* rows, int32_t n, int32_t q_heads,
+                int32_t kv_heads, int32_t head_dim, int32_t page_size, int64_t arena_rows,
+                int32_t layout, int32_t rope_dims, const float* inv_freq, void* stream) {
+  AppendParams prm;
+  if (const int rc = append_params(q, q_out, k, v, k_arena, v_arena, k_scale, v_scale, q8,
+                                   positions, rows, n, q_heads, kv_heads, head_dim, page_size,
+                                   arena_rows, layout, rope_dims, inv_freq, prm);
+      rc != PDA_OK || prm.hq + prm.hkv == 0)
+    return rc;
   void* args[] = {&prm};
-  const dim3 grid(n, (hq + hkv + kHeadsPerGroup - 1) / kHeadsPerGroup);
+  const dim3 grid(n, (prm.hq + prm.hkv + kHeadsPerGroup - 1) / kHeadsPerGroup);
   const void* fn = q8     ? reinterpret_cast<const void*>(rope_append_q8_kernel)
                    : bf16_elems ? reinterpret_cast<const void*>(rope_append_kernel<bf16>)
                           : reinterpret_cast<const void*>(rope_append_kernel<f16>);
@@ -275,6 +335,49 @@ int rope_append(const void* q, void* q_out, const void* k, const void* v, void* 
                                          static_cast<hipStream_t>(stream));
   if (err != hipSuccess)
     return fail(PDA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
+  return ok();
+}
+
+int rope_append_layers(const pda_append_layer* layers, int32_t num_layers, bool q8,
+                       bool bf16_elems, const int32_t* positions, const int32_t* rows, int32_t n,
+                       int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t page_size,
+                       int32_t layout, int32_t rope_dims, const float* inv_freq, void* stream) {
+  if (num_layers < 0 || (num_layers > 0 && !layers))
+    return fail(PDA_ERR_INVALID_ARGUMENT, "num_layers=%d layers=%p", num_layers,
+                static_cast<const void*>(layers));
+  if (q8 && bf16_elems)
+    return fail(PDA_ERR_INVALID_ARGUMENT, "8-bit arenas are written from fp16");
+  // Everything is checked before the first launch.
+  AppendLayersParams a = {};
+  for (int i = 0; i < num_layers; ++i) {
+    const pda_append_layer& l = layers[i];
+    if (!l.k || (l.q != nullptr) != (layers[0].q != nullptr))
+      return fail(PDA_ERR_INVALID_ARGUMENT,
+                  "every layer writes K/V, and all or none have queries (layer %d)", i);
+    if (const int rc = append_params(l.q, l.q_out, l.k, l.v, l.k_arena, l.v_arena, l.key_scales,
+                                     l.value_scales, q8, positions, rows, n, q_heads, kv_heads,
+                                     head_dim, page_size, l.arena_rows, layout, rope_dims,
+                                     inv_freq, a.common);
+        rc != PDA_OK)
+      return rc;
+  }
+  if (num_layers == 0 || n == 0) return ok();
+  const void* fn =
+      q8           ? reinterpret_cast<const void*>(rope_append_layers_kernel<f16, true>)
+      : bf16_elems ? reinterpret_cast<const void*>(rope_append_layers_kernel<bf16, false>)
+                   : reinterpret_cast<const void*>(rope_append_layers_kernel<f16, false>);
+  const unsigned groups =
+      (unsigned)((a.common.hq + a.common.hkv + kHeadsPerGroup - 1) / kHeadsPerGroup);
+  for (int first = 0; first < num_layers; first += kMaxLayers) {
+    const int count = num_layers - first < kMaxLayers ? num_layers - first : kMaxLayers;
+    for (int i = 0; i < count; ++i) a.layers[i] = layers[first + i];
+    void* args[] = {&a};
+    const hipError_t err =
+        hipLaunchKernel(fn, dim3((unsigned)n, groups, (unsigned)count), dim3(kAppendThreads),
+                        args, 0, static_cast<hipStream_t>(stream));
+    if (err != hipSuccess)
+      return fail(PDA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
+  }
   return ok();
 }
 
@@ -313,6 +416,18 @@ int pda_rope_append_q8(const void* q, void* q_out, const void* k, const void* v,
   return rope_append(q, q_out, k, v, k_arena, v_arena, key_scales, value_scales, true, false,
                      positions, rows, n, q_heads, kv_heads, head_dim, page_size, arena_rows,
                      layout, rope_dims, inv_freq, stream);
+}
+
+int pda_rope_append_layers(const pda_append_layer* layers, int32_t num_layers, int32_t kv_bits,
+                           int32_t bf16_elems, const int32_t* positions, const int32_t* rows,
+                           int32_t n, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+                           int32_t page_size, int32_t layout, int32_t rope_dims,
+                           const float* inv_freq, void* stream) {
+  if (kv_bits != 8 && kv_bits != 16)
+    return fail(PDA_ERR_INVALID_ARGUMENT, "kv_bits %d must be 8 or 16", kv_bits);
+  return rope_append_layers(layers, num_layers, kv_bits == 8, bf16_elems != 0, positions, rows, n,
+                            q_heads, kv_heads, head_dim, page_size, layout, rope_dims, inv_freq,
+                            stream);
 }
 
 }  // extern "C"

@@ -93,6 +93,20 @@ SIGNATURES["pda_rope_append_q8"] = (
 )
 
 
+class AppendLayer(ctypes.Structure):
+    """``pda_append_layer`` (pda.h): one layer's buffers of a step's append."""
+
+    _fields_ = [(name, c_void_p) for name in (
+        "q", "q_out", "k", "v", "k_arena", "v_arena", "key_scales", "value_scales")
+    ] + [("arena_rows", c_int64)]
+
+
+SIGNATURES["pda_rope_append_layers"] = (
+    ctypes.c_int,
+    [ctypes.POINTER(AppendLayer)] + [c_int32] * 3 + [c_void_p] * 2 + [c_int32] * 7
+    + [c_void_p] * 2,
+)
+
 
 class DecodeInfo(ctypes.Structure):
     """``pda_decode_info`` (pda.h): what a decode call of a shape launches."""

@@ -29,6 +29,7 @@ from __future__ import annotations
 import ctypes
 import os
 from collections import OrderedDict
+from collections.abc import Sequence
 from typing import Any
 
 import numpy as np
@@ -339,29 +340,9 @@ def _int32_vector(name: str, t: torch.Tensor, n: int) -> torch.Tensor:
     return t.contiguous()
 
 
-def rope_append(q: torch.Tensor | None, k: torch.Tensor, v: torch.Tensor,
-                keys: torch.Tensor, values: torch.Tensor, positions: torch.Tensor,
-                rows: torch.Tensor, *, page_size: int, dims: int, base: float | None = None,
-                freqs: Any = None, q_out: torch.Tensor | None = None,
-                scales: tuple[torch.Tensor, torch.Tensor] | None = None
-                ) -> torch.Tensor | None:
-    """Rotate this step's queries and keys and write the rotated keys and the
-    values into the arena, in one launch: the reference's
-    ``q = batch.rope(q, dims, ...)``, ``k = batch.rope(k, dims, ...)``
-    (batches.py:195-201) then ``cache.write(layer, rows, k, v)``
-    (batches.py:203-207, paged_kv.py:278-283).
-
-    ``q`` ``[n, q_heads, D]`` (or None), ``k``, ``v`` ``[n, kv_heads, D]``
-    fp16, or all bf16 (bf16 models: the rotation is rounded to bf16);
-    ``keys``/``values`` one layer's arena in either layout, of that dtype;
-    ``positions`` and ``rows`` int32 ``[n]`` (rows outside the arena are not
-    written). ``dims`` = 0 writes without rotation. Returns the rotated
-    queries (``q_out``, new unless given; ``q_out`` may be ``q``).
-
-    ``scales`` = (key_scales, value_scales) writes 8-bit K/V: ``keys`` and
-    ``values`` are int8 arenas, the rotated keys and the values are quantized
-    per (row, kv head) as ``paged_kv.quantize`` does (paged_kv.py:50-55);
-    the 8-bit write takes fp16 ``q``, ``k`` and ``v``."""
+def _check_append(q, k, v, keys, values, q_out, scales, page_size):
+    """The shape, type and layout checks of one layer's append; its geometry
+    and the rotated queries' buffer."""
     n, kv_heads, head_dim = (int(x) for x in k.shape)
     layout, arena_rows, a_heads, a_dim = _arena_geometry(keys, page_size)
     bf16 = k.dtype == torch.bfloat16 and scales is None
@@ -397,6 +378,34 @@ def rope_append(q: torch.Tensor | None, k: torch.Tensor, v: torch.Tensor,
         _check_half("q_out", q_out, 3, dtype)
         if q_out.shape != q.shape:
             raise ValueError("q_out must have q's shape")
+    return n, q_heads, kv_heads, head_dim, layout, arena_rows, bf16, q_out
+
+
+def rope_append(q: torch.Tensor | None, k: torch.Tensor, v: torch.Tensor,
+                keys: torch.Tensor, values: torch.Tensor, positions: torch.Tensor,
+                rows: torch.Tensor, *, page_size: int, dims: int, base: float | None = None,
+                freqs: Any = None, q_out: torch.Tensor | None = None,
+                scales: tuple[torch.Tensor, torch.Tensor] | None = None
+                ) -> torch.Tensor | None:
+    """Rotate this step's queries and keys and write the rotated keys and the
+    values into the arena, in one launch: the reference's
+    ``q = batch.rope(q, dims, ...)``, ``k = batch.rope(k, dims, ...)``
+    (batches.py:195-201) then ``cache.write(layer, rows, k, v)``
+    (batches.py:203-207, paged_kv.py:278-283).
+
+    ``q`` ``[n, q_heads, D]`` (or None), ``k``, ``v`` ``[n, kv_heads, D]``
+    fp16, or all bf16 (bf16 models: the rotation is rounded to bf16);
+    ``keys``/``values`` one layer's arena in either layout, of that dtype;
+    ``positions`` and ``rows`` int32 ``[n]`` (rows outside the arena are not
+    written). ``dims`` = 0 writes without rotation. Returns the rotated
+    queries (``q_out``, new unless given; ``q_out`` may be ``q``).
+
+    ``scales`` = (key_scales, value_scales) writes 8-bit K/V: ``keys`` and
+    ``values`` are int8 arenas, the rotated keys and the values are quantized
+    per (row, kv head) as ``paged_kv.quantize`` does (paged_kv.py:50-55);
+    the 8-bit write takes fp16 ``q``, ``k`` and ``v``."""
+    n, q_heads, kv_heads, head_dim, layout, arena_rows, bf16, q_out = _check_append(
+        q, k, v, keys, values, q_out, scales, page_size)
     rows = _int32_vector("rows", rows, n)
     if n == 0:
         return q_out
@@ -410,6 +419,44 @@ def rope_append(q: torch.Tensor | None, k: torch.Tensor, v: torch.Tensor,
                         arena_rows=arena_rows, layout=layout, dims=dims, table=table,
                         device=k.device, scales=scales, bf16=bf16)
     return q_out
+
+
+def rope_append_layers(q: Sequence[torch.Tensor], k: Sequence[torch.Tensor],
+                       v: Sequence[torch.Tensor], arenas: Sequence[tuple[torch.Tensor, ...]],
+                       positions: torch.Tensor, rows: torch.Tensor, *, page_size: int, dims: int,
+                       q_out: Sequence[torch.Tensor], base: float | None = None,
+                       freqs: Any = None) -> None:
+    """:func:`rope_append` of every layer of a step in one launch
+    (``pda_rope_append_layers``); ``arenas`` per layer ``(keys, values)`` or
+    ``(keys, values, key_scales, value_scales)``. The layers share the head
+    shape, the layout and the element types, and what one layer writes overlaps
+    nothing another layer reads or writes. Same bits as one call per layer."""
+    table = (_lib.AppendLayer * len(arenas))()
+    shared = None
+    for i, arena in enumerate(arenas):
+        scales = (arena[2], arena[3]) if len(arena) == 4 else None
+        n, *form, arena_rows, bf16, out = _check_append(q[i], k[i], v[i], arena[0], arena[1],
+                                                        q_out[i], scales, page_size)
+        form = (n, *form, bf16, scales is not None)
+        if shared is not None and form != shared:
+            raise ValueError("the layers of a step share shapes, layout and element types")
+        shared = form
+        buffers = (q[i], out, k[i], v[i], *arena) + (None,) * (4 - len(arena))
+        table[i] = _lib.AppendLayer(*(None if t is None else t.data_ptr() for t in buffers),
+                                    arena_rows)
+    if shared is None or shared[0] == 0:
+        return
+    n, q_heads, kv_heads, head_dim, layout, bf16, q8 = shared
+    rows = _int32_vector("rows", rows, n)
+    freq = None
+    if dims:
+        positions = _int32_vector("positions", positions, n)
+        freq = rope_inv_freq(dims, base=base, freqs=freqs, device=k[0].device)
+    rc = _lib.library().pda_rope_append_layers(
+        table, len(arenas), 8 if q8 else 16, int(bf16), positions.data_ptr() if dims else None,
+        rows.data_ptr(), n, q_heads, kv_heads, head_dim, page_size, layout, dims,
+        freq.data_ptr() if dims else None, torch.cuda.current_stream(k[0].device).cuda_stream)
+    _lib.check(rc)
 
 
 def rope(x: torch.Tensor, positions: torch.Tensor, dims: int, *, base: float | None = None,

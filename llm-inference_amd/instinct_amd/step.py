@@ -6,9 +6,9 @@ layer's ``rope`` + ``attend`` (:195-226) is launched separately, and its
 roadmap names the host-side step building as the limit on one user's decode
 speed (docs/roadmap.md:11-13,37). :class:`DecodeStepGraph` keeps the
 requests' page lists resident on the device (one row per request slot),
-packs them with one kernel (``pda_pack_decode_step``) and captures, for every
-layer, the fused RoPE + K/V append and the paged decode attention into one
-``torch.cuda.CUDAGraph`` (a HIP graph on ROCm). A step is then: write the
+packs them with one kernel (``pda_pack_decode_step``) and captures the fused
+RoPE + K/V append of all layers (one launch) and every layer's paged decode
+attention into one ``torch.cuda.CUDAGraph`` (a HIP graph on ROCm). A step is then: write the
 step's slots, positions and projected q/k/v into the static buffers, replay.
 Nothing of the step crosses PCIe except those inputs, and no kernel is
 launched from Python.
@@ -27,7 +27,7 @@ from typing import Any
 import torch
 
 from .hip_kernels import (decode_workspace_bytes, new_workspace, pack_decode_step,
-                          paged_decode_attention, rope_append)
+                          paged_decode_attention, rope_append, rope_append_layers)
 
 
 class DecodeStepGraph:
@@ -84,15 +84,37 @@ class DecodeStepGraph:
         pack_decode_step(self.seq_tables, self.slots, self.positions, width=self.width,
                          page_size=self.page_size, tables=self.tables, lengths=self.lengths,
                          rows=self.rows)
+        together = self._independent()
+        if together:
+            rope_append_layers(self.q, self.k, self.v, self.arenas, self.positions, self.rows,
+                               q_out=self.q_rot, page_size=self.page_size, **self.rope)
         for layer, arena in enumerate(self.arenas):
             keys, values = arena[0], arena[1]
             scales = (arena[2], arena[3]) if len(arena) == 4 else None
-            rope_append(self.q[layer], self.k[layer], self.v[layer], keys, values,
-                        self.positions, self.rows, q_out=self.q_rot[layer], scales=scales,
-                        page_size=self.page_size, **self.rope)
+            if not together:
+                rope_append(self.q[layer], self.k[layer], self.v[layer], keys, values,
+                            self.positions, self.rows, q_out=self.q_rot[layer], scales=scales,
+                            page_size=self.page_size, **self.rope)
             paged_decode_attention(self.q_rot[layer], keys, values, self.tables, self.lengths,
                                    out=self.out[layer], scales=scales,
                                    workspace=self.workspace, **self.kw)
+
+    def _independent(self) -> bool:
+        """Whether the appends of all layers may run before the first layer's
+        attention: the layers are of one form and no two buffers of the step
+        overlap (layers over one arena, or inputs that are another layer's
+        output, keep the order layer by layer)."""
+        if len({(len(a), a[0].dim(), a[0].dtype, q.shape, k.shape)
+                for a, q, k in zip(self.arenas, self.q, self.k)}) != 1:
+            return False
+        buffers = [self.slots, self.positions, self.tables, self.lengths, self.rows,
+                   self.seq_tables, self.workspace, *self.q, *self.k, *self.v, *self.q_rot,
+                   *self.out]
+        for arena in self.arenas:
+            buffers += arena
+        spans = sorted((t.data_ptr(), t.data_ptr() + t.numel() * t.element_size())
+                       for t in buffers if t.numel())
+        return all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
 
     def capture(self) -> None:
         """Capture :meth:`run` (after one eager run outside the capture).

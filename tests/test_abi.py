@@ -159,6 +159,24 @@ def test_append_validation_rejects_bad_arguments(overrides):
     assert _lib.library().pda_last_error()
 
 
+@pytest.mark.parametrize("overrides", [
+    dict(num_layers=-1), dict(layers=None), dict(kv_bits=4), dict(kv_bits=8),
+    dict(kv_bits=8, bf16=1), dict(n=-1), dict(head_dim=513), dict(rope_dims=3),
+    dict(layout=7), dict(rows=None), dict(positions=None), dict(second=dict(k=None)),
+    dict(second=dict(q=None, q_out=None)), dict(second=dict(arena_rows=0)),
+])
+def test_append_layers_validation_rejects_bad_arguments(overrides):
+    layer = dict(q=FAKE, q_out=FAKE, k=FAKE, v=FAKE, k_arena=FAKE, v_arena=FAKE, arena_rows=4096)
+    table = (_lib.AppendLayer * 2)(_lib.AppendLayer(**layer),
+                                   _lib.AppendLayer(**{**layer, **overrides.pop("second", {})}))
+    args = dict(layers=table, num_layers=2, kv_bits=16, bf16=0, positions=FAKE, rows=FAKE, n=4,
+                q_heads=28, kv_heads=4, head_dim=128, page_size=16,
+                layout=_lib.PDA_LAYOUT_PAGES, rope_dims=128, inv_freq=FAKE, stream=None)
+    args.update(overrides)
+    rc = _lib.library().pda_rope_append_layers(*args.values())
+    assert rc == _lib.PDA_ERR_INVALID_ARGUMENT
+
+
 def test_append_alignment_and_empty_calls():
     assert append(k=FAKE + 1) == _lib.PDA_ERR_ALIGNMENT
     assert append(rows=FAKE + 2) == _lib.PDA_ERR_ALIGNMENT
