@@ -347,7 +347,8 @@ constexpr int64_t kLocalMaxUnitBytes = int64_t(3) << 19;  // 1.5 MiB
 constexpr size_t kLocalMaxLds = size_t(64) << 10;
 
 size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, int page_size,
-                 int waves, int ring, int grid_pairs) {
+                 int waves, int ring, int grid_groups) {
+  const int grid_pairs = grid_groups * (waves / 2);
   const size_t lds = (size_t)pda_decode::local_lds_offset(batch) * sizeof(int32_t) +
                      (size_t)waves * pl.unit_heads * (dim * sizeof(float) + sizeof(float2));
   if (lds > kLocalMaxLds) return 0;
@@ -364,6 +365,26 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, int
       1, std::min<int64_t>(grid_pairs, (pl.pages_est + 2 * pl.min_pages - 1) /
                                            (2 * pl.min_pages)));
   const bool short_waves = 16 * pl.unit_pages_max * pairs <= 5 * ring * waves * pl.pages_est;
+  // A short unit costs its workgroup less than the stream's second launch and
+  // dependent trips, however few pages the stream gives a wave. Local / stream,
+  // us a call among others: 32/8 heads of 128, 4 x 512 keys 11.8 / 15.6,
+  // 4 x 768 14.7 / 16.9, 4 x 1024 17.4 / 17.4; 14/2 of 64, 1 x 512 11.1 / 14.8,
+  // 1 x 1024 16.1 / 11.6; on the matrix cores (a wave takes one page at a time)
+  // 28/4 of 128, 1 x 384 13.7 / 14.1, 1 x 512 15.2 / 14.3; one head a unit,
+  // 32/32 of 80, 1 x 384 10.3 / 11.5, 1 x 768 14.0 / 12.0; 8/4 of 256,
+  // 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0. Units past the resident
+  // workgroups keep the rule above.
+  const int64_t unit_keys = pl.unit_pages_max * page_size;
+  const int64_t short_keys = dim > 128  ? 256
+                             : dim <= 64 ? 768
+                             : pl.mf || pl.unit_heads == 1 ? 384
+                                                           : 768;
+  if (units <= grid_groups && unit_keys <= short_keys) return lds;
+  // More units than resident workgroups, of several heads: the stream's even
+  // split wins back its second launch (32/8 heads, 64 sequences of 256 keys,
+  // stream / local: 23.1 / 25.7 at head dim 128, 24.7 / 31.8 at 96, 20.1 / 21.7
+  // at 8 bits; of 64 keys level; two heads of 256 level).
+  if (units > grid_groups && pl.unit_heads > 2 && pl.unit_pages_max > waves) return 0;
   return units <= kLocalMaxUnits && unit_bytes <= kLocalMaxUnitBytes && short_waves ? lds : 0;
 }
 
@@ -494,7 +515,7 @@ int plan_launch(Plan& pl, int32_t batch, int32_t kv_heads, int32_t head_dim,
   const int grid_pairs = lp.groups * (lp.kp.split_waves / 2);
   lp.dim = pl.mf ? head_dim : kernel_dim(head_dim, q8);
   lp.lds_local = local_lds(pl, batch, kv_heads, lp.dim, q8 ? 1 : 2, page_size,
-                           lp.kp.split_waves, lp.kp.ring, grid_pairs);
+                           lp.kp.split_waves, lp.kp.ring, lp.groups);
   // Local mode on the VALU kernels, when a unit per GQA group leaves CUs
   // idle: a unit per query head, as long as the units still fit one
   // workgroup per resident slot. The units of one kv head read the same
