@@ -306,7 +306,7 @@ struct MergeShape {
   int waves;   // per workgroup
 };
 
-MergeShape merge_shape(const Plan& pl, int dim, int grid_pairs, int64_t heads) {
+MergeShape merge_shape(const Plan& pl, int dim, bool gen, int grid_pairs, int64_t heads) {
   const int64_t pairs = std::max<int64_t>(
       1, std::min<int64_t>(grid_pairs, (pl.pages_est + 2 * pl.min_pages - 1) /
                                            (2 * pl.min_pages)));
@@ -319,9 +319,18 @@ MergeShape merge_shape(const Plan& pl, int dim, int grid_pairs, int64_t heads) {
     const char* e = getenv("PDA_MERGE_SLICED");
     return e && *e ? atoi(e) : -1;
   }();
+  // The sliced kernel reads each piece's (max, sum) once instead of on every
+  // lane, so at the head dims whose rows need few slices it is also the faster
+  // one for fewer pieces (us a call, whole rows / sliced: 14/2 heads of 64,
+  // 1 x 768 keys 15.1 / 11.0, 64 x 512 23.1 / 19.1; 28/4 of 128, 1 x 768
+  // 14.6 / 13.1, 16 x 1024 20.1 / 18.6; 4 x 64 level, 64 x 64 16.2 / 16.8;
+  // slower at 256 and the generic dims: 8/4 of 256, 16 x 256 14.4 / 15.1;
+  // 32/32 of 80, 16 x 256 18.2 / 19.1).
+  const bool narrow = !gen && heads * chunks <= 1024 &&
+                      ((dim == 64 && pieces >= 8) || (dim == 128 && pieces >= 14));
   const bool sliced = force >= 0 ? force > 0
-                                 : pieces > kMergeSlicedRound &&
-                                       heads * chunks <= kMergeSlicedMaxGroups;
+                                 : (pieces > kMergeSlicedRound &&
+                                    heads * chunks <= kMergeSlicedMaxGroups) || narrow;
   const int per_round = sliced ? kMergeSlicedRound : 32 / chunks;
   const int64_t mw = (pieces + per_round - 1) / per_round;
   return {sliced, sliced ? chunks : 1,
@@ -366,19 +375,23 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, int
                                            (2 * pl.min_pages)));
   const bool short_waves = 16 * pl.unit_pages_max * pairs <= 5 * ring * waves * pl.pages_est;
   // A short unit costs its workgroup less than the stream's second launch and
-  // dependent trips, however few pages the stream gives a wave. Local / stream,
-  // us a call among others: 32/8 heads of 128, 4 x 512 keys 11.8 / 15.6,
-  // 4 x 768 14.7 / 16.9, 4 x 1024 17.4 / 17.4; 14/2 of 64, 1 x 512 11.1 / 14.8,
-  // 1 x 1024 16.1 / 11.6; on the matrix cores (a wave takes one page at a time)
-  // 28/4 of 128, 1 x 384 13.7 / 14.1, 1 x 512 15.2 / 14.3; one head a unit,
-  // 32/32 of 80, 1 x 384 10.3 / 11.5, 1 x 768 14.0 / 12.0; 8/4 of 256,
+  // dependent trips, however few pages the stream gives a wave; the line lies
+  // higher from 64 units on, where the stream has more to merge. Local /
+  // stream, us a call among others: 14/2 heads of 64, 1 x 384 keys 10.1 / 10.9,
+  // 1 x 768 13.5 / 11.0, 64 x 512 12.5 / 19.1; 32/8 of 128, 1 x 512 11.4 / 13.5,
+  // 1 x 768 14.2 / 13.6, 16 x 768 19.7 / 20.3; of 96, 1 x 768 14.6 / 17.3; on the matrix cores (a wave takes
+  // one page at a time) 28/4 of 128, 1 x 256 11.5 / 12.8, 1 x 384 13.7 / 13.1,
+  // 16 x 512 16.3 / 17.7, 16 x 768 20.0 / 17.9; one head a unit, 32/32 of 80,
+  // 1 x 384 10.3 / 11.5, 1 x 768 14.0 / 12.0, 4 x 768 15.0 / 17.2; 8/4 of 256,
   // 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0. Units past the resident
   // workgroups keep the rule above.
   const int64_t unit_keys = pl.unit_pages_max * page_size;
-  const int64_t short_keys = dim > 128  ? 256
-                             : dim <= 64 ? 768
-                             : pl.mf || pl.unit_heads == 1 ? 384
-                                                           : 768;
+  const bool many = units >= 64;
+  const int64_t short_keys = dim > 128              ? 256
+                             : dim <= 64            ? (many ? 768 : 512)
+                             : pl.mf                ? (many ? 512 : 320)
+                             : pl.unit_heads == 1   ? (many ? 768 : 384)
+                                                    : (many || dim < 128 ? 768 : 640);
   if (units <= grid_groups && unit_keys <= short_keys) return lds;
   // More units than resident workgroups, of several heads: the stream's even
   // split wins back its second launch (32/8 heads, 64 sequences of 256 keys,
@@ -542,7 +555,7 @@ int plan_launch(Plan& pl, int32_t batch, int32_t kv_heads, int32_t head_dim,
     }
   }
   const int heads = kv_heads * pl.nhg * pl.unit_heads;
-  lp.ms = merge_shape(pl, lp.dim, grid_pairs, (int64_t)heads * batch);
+  lp.ms = merge_shape(pl, lp.dim, lp.kp.gen, grid_pairs, (int64_t)heads * batch);
   *out = lp;
   return PDA_OK;
 }
