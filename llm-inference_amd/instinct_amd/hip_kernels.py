@@ -50,7 +50,8 @@ def new_workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
 
 
-def stream_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
+def stream_workspace(device: torch.device, nbytes: int,
+                     stream: int | None = None) -> torch.Tensor:
     """A cached, 256-byte aligned device workspace of at least ``nbytes``
     for the current stream of ``device``, grown on demand and
     shared by calls of any shape on that stream (calls on one stream never
@@ -65,7 +66,9 @@ def stream_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     pass a workspace it owns instead (``workspace=`` of the calls), as
     :class:`instinct_amd.step.DecodeStepGraph` does."""
     index = device.index if device.index is not None else torch.cuda.current_device()
-    key = (index, int(torch.cuda.current_stream(index).cuda_stream))
+    if stream is None:  # (a caller that has the current stream's handle passes it)
+        stream = int(torch.cuda.current_stream(index).cuda_stream)
+    key = (index, stream)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         size = max(nbytes, 1 << 20)
@@ -175,7 +178,7 @@ def paged_decode_attention(
     takes their dtype, as the reference's quantized kernel does
     (metal_kernels.py:196-206)."""
     q8 = scales is not None
-    batch, q_heads, head_dim = (int(n) for n in queries.shape)
+    batch, q_heads, head_dim = queries.shape
     kv_heads = int(keys.shape[1])
     if keys.dim() == 3:
         layout, arena_rows, width = _lib.PDA_LAYOUT_ROWS, int(keys.shape[0]), int(keys.shape[2])
@@ -210,7 +213,7 @@ def paged_decode_attention(
                 raise ValueError(f"{name} must be float16 {list(scale_shape)}")
             if not t.is_cuda or not t.is_contiguous():
                 raise ValueError(f"{name} must be a contiguous GPU tensor")
-    if tuple(keys.shape) != tuple(values.shape) or width != head_dim:
+    if keys.shape != values.shape or width != head_dim:
         raise ValueError("keys and values must have the same shape and head_dim")
     if tables.dtype != torch.int32 or lengths.dtype != torch.int32:
         raise TypeError("tables and lengths must be int32")
@@ -226,10 +229,10 @@ def paged_decode_attention(
     stride = int(tables.shape[1])
     need = _lib.workspace_bytes(batch, q_heads, kv_heads, head_dim, page_size, stride,
                                 int(longest), int(window), int(split_pages))
-    ws = (stream_workspace(device, need) if workspace is None
+    stream = int(torch.cuda.current_stream(device).cuda_stream)
+    ws = (stream_workspace(device, need, stream) if workspace is None
           else _given_workspace(workspace, device, need))
-    stream = torch.cuda.current_stream(device).cuda_stream
-    if out.dtype != q_dtype or tuple(out.shape) != tuple(queries.shape) or not out.is_cuda:
+    if out.dtype != q_dtype or out.shape != queries.shape or not out.is_cuda:
         raise ValueError("out must match the queries' shape and dtype")
     entry = {"both": "pda_paged_decode_attention", "split": "pda_decode_split",
              "merge": "pda_decode_merge"}[passes] + ("_q8" if q8 else "") + ("_bf16" if bf16 else "")
@@ -240,7 +243,7 @@ def paged_decode_attention(
         int(page_size), stride, arena_rows, layout, int(longest), float(scale),
         int(window), float(softcap), int(split_pages),
         0 if deterministic else _lib.PDA_DECODE_RACING, ws.data_ptr(),
-        ws.numel(), ctypes.c_void_p(stream))
+        ws.numel(), stream)
     _lib.check(rc)
     return out
 
