@@ -175,10 +175,14 @@ __device__ __forceinline__ void copy_to_lds(const void* src, uint32_t dst) {
 }
 
 // The same product added to c; kAcc: c in accumulator registers, which the
-// compiler would otherwise copy to vector registers and back. (The compiler
-// does not know what such an instruction still has in flight: c is only read
-// by further ones until outputs_done; s_nop: operands a VALU instruction has
-// just written.)
+// compiler would otherwise copy to vector registers and back. The compiler
+// neither knows what such an instruction still has in flight nor that its
+// operands need two wait states after a VALU instruction wrote them. So c is
+// only read by further products until outputs_done, the weights pass through
+// operands_done after they were last written, and the fragments come from LDS.
+// (Two wait states in front of every product instead: 565 against 556 us for
+// 4096 tokens at 8192, 28/4 heads of 128.) A test reads the distances from the
+// built kernels.
 template <bool BF, bool kAcc>
 __device__ __forceinline__ void mfma_to(const f16x8& a, const f16x8& b, f32x16& c) {
   if constexpr (!kAcc)
@@ -1157,6 +1161,15 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       }
     }
   };
+  // Between the last write of a block's weights and the first product that
+  // reads them. (The outputs' rescaling lies before the weights' in settle.)
+  auto operands_done = [&](f16x8 (&pb)[QB][2]) {
+    if constexpr (kAcc) {
+#pragma unroll
+      for (int j = 0; j < QB; ++j) asm volatile("" : "+v"(pb[j][0]), "+v"(pb[j][1]));
+      asm volatile("s_nop 1");
+    }
+  };
   // Before the outputs are read by anything but a matrix-core instruction.
   auto outputs_done = [&]() {
     if constexpr (kAcc) {
@@ -1200,6 +1213,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
                    __builtin_amdgcn_exp2f(fmaf(x[2 * i + 1], c, -mu)));
         lb[j] = total(pb[j], 0.0f);
       }
+      operands_done(pb);
     }
 #pragma unroll
     for (int j = 0; j < QB; ++j) l[j] += lb[j];
@@ -1277,6 +1291,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
 #pragma unroll
       for (int b = 0; b < (kAcc ? 0 : D / 32); ++b) asm volatile("" : "+v"(o[j][b]));
     }
+    operands_done(pb);
   };
 
   // Whether the blocks of an iteration (the odd one of the tile before and
@@ -1380,6 +1395,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       unweighed();
       settle(s1, p1, lb);
       accumulate(p1, vt + 1024);
+      outputs_done();  // (here: copies of the outputs may follow on any way out)
       if (t < t_end) {
         turn();
         close(t, ok);
@@ -1387,7 +1403,6 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
     }
     for (++t; t < t_end; ++t) idle();
   }
-  outputs_done();
 #pragma unroll
   for (int j = 0; j < QB; ++j)
     finish<D, BF, false, false>(p, o[j], m[j], l[j], qi + 32 * j, h, split, hh, 0,
