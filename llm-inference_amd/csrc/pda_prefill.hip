@@ -629,8 +629,12 @@ __device__ __forceinline__ void prefill_body(const PrefillParams p) {
 
   int page0, r0, s0, page1, r1, s1;
   bool in0, in1;
-  lookup(page0, in0, r0, s0);
-  lookup(page1, in1, r1, s1);
+  page0 = page1 = r0 = r1 = s0 = s1 = 0;
+  in0 = in1 = false;
+  // Only tiles of the range are looked up: the key after them may be 2^31,
+  // past what the cursor holds.
+  if (t_begin < t_end) lookup(page0, in0, r0, s0);
+  if (t_begin + 1 < t_end) lookup(page1, in1, r1, s1);
   fetch(page0, in0, r0, s0);
   stash(0);
   if constexpr (kOneV) stash_v(0);
@@ -645,7 +649,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams p) {
     if constexpr (kOneV)
       if (t > t_begin) stash_v(0);
     if (more) fetch(page1, in1, r1, s1);
-    lookup(page1, in1, r1, s1);
+    if (t + 2 < t_end) lookup(page1, in1, r1, s1);
 
     const bool work = wave_live && k0 <= wave_last &&
                       (p.window <= 0 || wave_img || k0 + kKeys - 1 > wfirst - p.window);
@@ -985,9 +989,11 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
 
   // Gather: thread tid moves key tid / 4 of a tile, 64-byte pieces.
   const int gk = tid >> 2;
-  int kp = kbase + t_begin * kKeys + gk;
-  int pi = kp / p.page_size;
-  int r = kp - pi * p.page_size;
+  // Unsigned: the cursors run past the last key, which may be 2^31 - 2.
+  const uint32_t page_size = p.page_size, table_len = p.table_len;
+  uint32_t kp = (uint32_t)kbase + (uint32_t)(t_begin * kKeys) + gk;
+  uint32_t pi = kp / page_size;
+  uint32_t r = kp - pi * page_size;
   // 16-byte chunk of each 64-byte piece this lane fetches: K's are swizzled.
   const int kchunk = 8 * ((lane & 3) ^ ((lane >> 4) & 3));
   const int vchunk = 8 * (lane & 3);
@@ -998,26 +1004,26 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
   // 64 keys of the tile as well (one per lane) for the mask of usable keys,
   // which then needs neither LDS nor a barrier.
   const uint32_t pages = (uint32_t)min(p.arena_pages, (int64_t)INT32_MAX);
-  const int step_pages = kKeys / p.page_size, step_rows = kKeys % p.page_size;
+  const uint32_t step_pages = kKeys / page_size, step_rows = kKeys % page_size;
   int page = 0, row_off = 0, page_m = 0;
   bool in = false, in_m = false;
-  int kp_m = kbase + t_begin * kKeys + lane;
-  int pi_m = kp_m / p.page_size;
-  int r_m = kp_m - pi_m * p.page_size;
+  uint32_t kp_m = kp - gk + lane;
+  uint32_t pi_m = kp_m / page_size;
+  uint32_t r_m = kp_m - pi_m * page_size;
   auto lookup = [&]() {
-    in = kp <= last && pi < p.table_len;
-    in_m = kp_m <= last && pi_m < p.table_len;
-    page = p.table[min(pi, p.table_len - 1)];
-    page_m = p.table[min(pi_m, p.table_len - 1)];
-    row_off = r * p.row_elems + kvh * p.head_elems;
+    in = kp <= (uint32_t)last && pi < table_len;
+    in_m = kp_m <= (uint32_t)last && pi_m < table_len;
+    page = p.table[min(pi, table_len - 1)];
+    page_m = p.table[min(pi_m, table_len - 1)];
+    row_off = (int)r * p.row_elems + kvh * p.head_elems;
     kp += kKeys;
     kp_m += kKeys;
     r += step_rows;
     r_m += step_rows;
-    pi += step_pages + (r >= p.page_size ? 1 : 0);
-    pi_m += step_pages + (r_m >= p.page_size ? 1 : 0);
-    r -= r >= p.page_size ? p.page_size : 0;
-    r_m -= r_m >= p.page_size ? p.page_size : 0;
+    pi += step_pages + (r >= page_size ? 1 : 0);
+    pi_m += step_pages + (r_m >= page_size ? 1 : 0);
+    r -= r >= page_size ? page_size : 0;
+    r_m -= r_m >= page_size ? page_size : 0;
   };
   // This thread's rows of the tiles whose V and K are copied next, their
   // usable keys, and those of the tile after them.
@@ -1298,9 +1304,9 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
   // the even one of this tile) need their masks, a softcap or an unusual scale.
   const bool special = p.softcap > 0.0f || !(p.scale_log2 > 0.0f);
   const int plain_hi = special ? INT32_MIN : wfirst - 31;
-  const int plain_lo = p.window > 0 ? wlast - p.window + 32 : INT32_MIN;
+  const int plain_lo = p.window > 0 ? wlast - p.window : INT32_MIN;
   auto rough = [&](int k0) {
-    return k0 > plain_hi || k0 <= plain_lo || ((ok_prev >> 32) & (uint32_t)ok_now) != 0xFFFFFFFFu;
+    return k0 > plain_hi || k0 - 32 <= plain_lo || ((ok_prev >> 32) & (uint32_t)ok_now) != 0xFFFFFFFFu;
   };
   // Iteration t of the workgroup: V of tile t and K of tile t + 1 are copied
   // beside the iteration's math and published by its barrier (close). The
@@ -1390,7 +1396,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       const uint32_t ok_odd = (uint32_t)(ok_prev >> 32);
       if (t < t_end) copies(t);
       const f16* vt = s_v[((t - t_begin) & 1) ^ 1];
-      shape(s1, kbase + t * kKeys - 32, ok_odd);
+      shape(s1, kbase + (t - 1) * kKeys + 32, ok_odd);
       accumulate(p0, vt);
       unweighed();
       settle(s1, p1, lb);
