@@ -178,8 +178,9 @@ __device__ __forceinline__ void copy_to_lds(const void* src, uint32_t dst) {
 // compiler would otherwise copy to vector registers and back. The compiler
 // neither knows what such an instruction still has in flight nor that its
 // operands need two wait states after a VALU instruction wrote them. So c is
-// only read by further products until outputs_done, the weights pass through
-// operands_done after they were last written, and the fragments come from LDS.
+// only read by further products until outputs_done, the weights' sum or
+// operands_done comes between their last write and the first product that reads
+// them, and the fragments come from LDS.
 // (Two wait states in front of every product instead: 565 against 556 us for
 // 4096 tokens at 8192, 28/4 heads of 128.) A test reads the distances from the
 // built kernels.
@@ -1167,8 +1168,9 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       }
     }
   };
-  // Between the last write of a block's weights and the first product that
-  // reads them. (The outputs' rescaling lies before the weights' in settle.)
+  // Between the re-weighing of a block and the first product that reads the
+  // weights. (The outputs' rescaling lies before it. Weights that a step has
+  // taken need no wait: their sum, pinned with them, comes after.)
   auto operands_done = [&](f16x8 (&pb)[QB][2]) {
     if constexpr (kAcc) {
 #pragma unroll
@@ -1297,7 +1299,6 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
 #pragma unroll
       for (int b = 0; b < (kAcc ? 0 : D / 32); ++b) asm volatile("" : "+v"(o[j][b]));
     }
-    operands_done(pb);
   };
 
   // Whether the blocks of an iteration (the odd one of the tile before and
