@@ -165,7 +165,7 @@ __device__ __forceinline__ uint32_t lds_address(const void* at) {
 // 16 bytes per lane from global memory straight into LDS: lane i's, from src +
 // kOff bytes, to dst + kOff + kPlus + 16 i (dst: wave-uniform; the
 // instruction adds its offset to both addresses). The caller waits
-// (wait_vmem0) before the barrier that publishes them.
+// (wait_vmem) before the barrier that publishes them.
 template <int kOff, int kPlus>
 __device__ __forceinline__ void copy_to_lds(const void* src, uint32_t dst) {
   asm volatile("s_add_u32 m0, %0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%3" ::"s"(
@@ -200,7 +200,12 @@ __device__ __forceinline__ void each(F& f, std::integer_sequence<int, kI...>) {
   (f(std::integral_constant<int, kI>{}), ...);
 }
 
-__device__ __forceinline__ void wait_vmem0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// Until at most kLeft of the wave's loads and copies are under way.
+template <int kLeft>
+__device__ __forceinline__ void wait_vmem() {
+  static_assert(kLeft < 64, "the count has six bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (kLeft & 15) | (kLeft >> 4) << 14);
+}
 
 // Output of one query: normalised, or the unnormalised partial of a key range.
 template <int D, bool BF, bool GEN, bool ODD>
@@ -892,6 +897,11 @@ __device__ __forceinline__ void prefill_body(const PrefillParams p) {
 // 32256 1.14 PFLOP/s. D = 64 (14/2 heads, 1531 at 389): 30.8 -> 26.0 us. D = 256
 // (16/8 heads, 2048 at 6144, window 1024): 80 -> 59 us.
 //
+// Short calls: the queries' loads, the table entries and the first tiles' copies
+// are under way together, a 32-key block past a wave's last key is left out, and
+// outputs that are still zeros are not rescaled. 16/8 heads of 256, 19 tokens at
+// 0: 6.8 us; 9.6 with the loads in a row, both blocks always and the rescaling.
+//
 // Measured and not kept: the weights' sum on v_dot2 inside the step (each
 // holds the matrix pipe for 18 cycles: step 1,156 against 1,040), fp32 adds
 // of the rounded weights instead (level), operands read 2, 4 or 5 ahead
@@ -954,8 +964,6 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
     for (int c = 0; c < D / 16; ++c) {
       const f16x8 x = *reinterpret_cast<const f16x8*>(qp + 16 * c);
       qf[j][c] = live ? x : f16x8{};
-      // (Only ever matrix-core operands.)
-      if constexpr (kAcc) asm volatile("" : "+a"(qf[j][c]));
     }
   }
 
@@ -1206,13 +1214,18 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
         for (int v = 1; v < 16; ++v) top = fmaxf(top, x[v]);
         top = fmaxf(top, __shfl_xor(top, 32)) * c;
         if (top > m[j] + kSlack) {
-          const float f = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - top);
+          const bool seen = m[j] != -INFINITY;
+          const float f = seen ? __builtin_amdgcn_exp2f(m[j] - top) : 0.0f;
           m[j] = top;
-          l[j] *= f;
+          // (Else the outputs are zeros. With two blocks the choice costs the loop
+          // its registers' order and 1%.)
+          if (QB == 2 || seen) {
+            l[j] *= f;
 #pragma unroll
-          for (int b = 0; b < D / 32; ++b)
+            for (int b = 0; b < D / 32; ++b)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) o[j][b][v] *= f;
+              for (int v = 0; v < 16; ++v) o[j][b][v] *= f;
+          }
         }
         const float mu = m[j] == -INFINITY ? 0.0f : m[j];
 #pragma unroll
@@ -1323,23 +1336,44 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
     each_plane([&](auto i) { copy_k(buf ^ 1, i); });
   };
   auto close = [&](int t, bool ok) {
-    wait_vmem0();
+    wait_vmem<0>();
     clean_v((t - t_begin) & 1, ok);
     __syncthreads();
   };
   int t = t_begin;
   lookup();
+  __builtin_amdgcn_sched_barrier(0);
+  // The queries are only ever matrix-core operands: into accumulator
+  // registers, while the table entries are on their way. (Moved one by one as
+  // they were loaded, each load waited for the one before.)
+  if constexpr (kAcc) {
+#pragma unroll
+    for (int j = 0; j < QB; ++j)
+#pragma unroll
+      for (int c = 0; c < D / 16; ++c) asm volatile("" : "+a"(qf[j][c]));
+  }
   advance();
   lookup();
-  each_plane([&](auto i) { copy_k(0, i); });
+  const f16* first_k = src_k;
   advance();
+  // (The second entries are waited for here: a wait past the first copies
+  // would wait for those as well.)
+  asm volatile("" : "+v"(first_k), "+v"(src_v), "+v"(src_k), "+s"(ok_next));
   lookup();
-  wait_vmem0();
+  // K of the first tile, then its V and the second K: only the first is
+  // waited for here, so a short call has one latency of K/V and not two.
+  each_plane([&](auto i) {
+    copy_to_lds<64 * i.value, (2 * kPlane - 64) * i.value>(first_k, k_dst);
+  });
+  copies(t);
+  wait_vmem<2 * kPlanes>();
   __syncthreads();
+  // Whether the odd block of the wave's last tile holds a key it sees.
+  const bool odd_last = wave_last >= kbase + (wb - 1) * kKeys + 32;
   if (wa >= wb) wa = t_end;
   auto idle = [&]() {  // an iteration whose tile this wave's queries do not see
     const bool ok = ok_v;
-    copies(t);
+    if (t > t_begin) copies(t);
     turn();
     close(t, ok);
   };
@@ -1353,12 +1387,12 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
     // First tile: scores of both blocks, weights of the first.
     {
       const bool ok = ok_v;
-      copies(t);
+      if (t > t_begin) copies(t);
       const f16* kt = s_k[(t - t_begin) & 1];
       const int k0 = kbase + t * kKeys;
       scores(s0, kt);
       shape(s0, k0, (uint32_t)ok_now);
-      scores(s1, kt + 1024);
+      if (wb - wa > 1 || odd_last) scores(s1, kt + 1024);
       unweighed();
       settle(s0, p0, lb);
       turn();
@@ -1397,11 +1431,13 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       const uint32_t ok_odd = (uint32_t)(ok_prev >> 32);
       if (t < t_end) copies(t);
       const f16* vt = s_v[((t - t_begin) & 1) ^ 1];
-      shape(s1, kbase + (t - 1) * kKeys + 32, ok_odd);
+      if (odd_last) shape(s1, kbase + (t - 1) * kKeys + 32, ok_odd);
       accumulate(p0, vt);
-      unweighed();
-      settle(s1, p1, lb);
-      accumulate(p1, vt + 1024);
+      if (odd_last) {
+        unweighed();
+        settle(s1, p1, lb);
+        accumulate(p1, vt + 1024);
+      }
       outputs_done();  // (here: copies of the outputs may follow on any way out)
       if (t < t_end) {
         turn();
@@ -1409,6 +1445,15 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       }
     }
     for (++t; t < t_end; ++t) idle();
+  }
+  // (An empty range has waited for none but its first copies; the others have
+  // to land before the LDS is another workgroup's.)
+  wait_vmem<0>();
+  // One block of outputs a wave leaves room for them in vector registers: moved
+  // at once, not each before its store (0.4 us).
+  if constexpr (kAcc && QB == 1) {
+#pragma unroll
+    for (int b = 0; b < D / 32; ++b) asm volatile("" : "+v"(o[0][b]));
   }
 #pragma unroll
   for (int j = 0; j < QB; ++j)
