@@ -1093,9 +1093,10 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
     const uint32_t ones = n >= 32 ? 32u : n > 0 ? (uint32_t)n : 0u;
     return (uint32_t)((1ull << ones) - 1);
   };
-  // Scores of a block in place: softcap or a scale that is not positive,
-  // then the masks.
-  auto shape = [&](f32x16 (&xs)[QB], int k0, uint32_t okm) {
+  // Scores of a block in place: softcap or a scale that is not positive
+  // (`special`), then the masks where the block has any.
+  const bool special = p.softcap > 0.0f || !(p.scale_log2 > 0.0f);
+  auto shape = [&](f32x16 (&xs)[QB], int k0, uint32_t okm, bool masks) {
 #pragma unroll
     for (int j = 0; j < QB; ++j) {
       f32x16& x = xs[j];
@@ -1109,6 +1110,11 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) x[v] = x[v] * p.scale_log2;
       }
+    }
+    if (!masks) return;
+#pragma unroll
+    for (int j = 0; j < QB; ++j) {
+      f32x16& x = xs[j];
       // Keys k0 .. k0 + 31 this lane's query sees, one bit each: usable, and
       // not past its position, inside its window, or inside its image. Two
       // instructions per score then (bit to mask, select), where a test of
@@ -1316,11 +1322,17 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
 
   // Whether the blocks of an iteration (the odd one of the tile before and
   // the even one of this tile) need their masks, a softcap or an unusual scale.
-  const bool special = p.softcap > 0.0f || !(p.scale_log2 > 0.0f);
   const int plain_hi = special ? INT32_MIN : wfirst - 31;
   const int plain_lo = p.window > 0 ? wlast - p.window : INT32_MIN;
   auto rough = [&](int k0) {
     return k0 > plain_hi || k0 - 32 <= plain_lo || ((ok_prev >> 32) & (uint32_t)ok_now) != 0xFFFFFFFFu;
+  };
+  // Whether a block needs its masks (every block of a softcapped call comes
+  // through the test above; masked as well, whatever its keys, 4096 tokens at
+  // 8192, 14/2 heads of 64, took 407 us instead of 367). One test in the loop:
+  // a second beside it cost two query blocks 2%.
+  auto masked = [&](int k0, uint32_t okm) {
+    return !special || k0 > wfirst - 31 || k0 <= plain_lo || okm != 0xFFFFFFFFu;
   };
   // Iteration t of the workgroup: V of tile t and K of tile t + 1 are copied
   // beside the iteration's math and published by its barrier (close). The
@@ -1391,7 +1403,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       const f16* kt = s_k[(t - t_begin) & 1];
       const int k0 = kbase + t * kKeys;
       scores(s0, kt);
-      shape(s0, k0, (uint32_t)ok_now);
+      shape(s0, k0, (uint32_t)ok_now, true);
       if (wb - wa > 1 || odd_last) scores(s1, kt + 1024);
       unweighed();
       settle(s0, p0, lb);
@@ -1406,8 +1418,8 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       const f16* kt = s_k[buf];
       const f16* vt = s_v[buf ^ 1];
       const bool masks = rough(k0), ok = ok_v;
-      const uint32_t ok_even = (uint32_t)ok_now;
-      if (masks) shape(s1, k0 - 32, (uint32_t)(ok_prev >> 32));
+      const uint32_t ok_even = (uint32_t)ok_now, ok_odd = (uint32_t)(ok_prev >> 32);
+      if (masks) shape(s1, k0 - 32, ok_odd, masked(k0 - 32, ok_odd));
       step(s1, p1, p0, s0, lb, kt, vt, [&](auto i) {
         if constexpr (i.value % 2 == 0) {
           constexpr int j = i.value / 2;
@@ -1418,7 +1430,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
         }
       });
       settle(s1, p1, lb);
-      if (masks) shape(s0, k0, ok_even);
+      if (masks) shape(s0, k0, ok_even, masked(k0, ok_even));
       step(s0, p0, p1, s1, lb, kt + 1024, vt + 1024, [&](auto i) {
         if constexpr (i.value == 1) turn();
       });
@@ -1431,7 +1443,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       const uint32_t ok_odd = (uint32_t)(ok_prev >> 32);
       if (t < t_end) copies(t);
       const f16* vt = s_v[((t - t_begin) & 1) ^ 1];
-      if (odd_last) shape(s1, kbase + (t - 1) * kKeys + 32, ok_odd);
+      if (odd_last) shape(s1, kbase + (t - 1) * kKeys + 32, ok_odd, true);
       accumulate(p0, vt);
       if (odd_last) {
         unweighed();
