@@ -61,8 +61,11 @@
 
 #include "pda.h"
 #include "pda_internal.h"
+#include "pda_prefill_plan.h"
 
 namespace {
+
+using namespace pda_prefill;
 
 typedef _Float16 f16;
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -78,17 +81,6 @@ typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr float kSlack = 8.0f;
-constexpr int kWaves = 4;  // waves per workgroup (D <= 256)
-// Waves that split the head dim: at D = 512 the query fragments and output
-// accumulators of 32 queries do not fit one wave's registers, so four waves
-// share 32 queries, each holding 128 dims of Q and O; a D = 512 workgroup has
-// eight waves (two such query blocks). (Split the same way, D = 256 runs two
-// waves per SIMD instead of one but was 2-5% slower: the score exchange
-// costs more than the second wave hides.)
-constexpr int slices_for(int d) { return d > 256 ? 4 : 1; }
-constexpr int waves_for(int d) { return d > 256 ? 2 * kWaves : kWaves; }
-// Queries per workgroup: 32 per query block.
-constexpr int queries_for(int d) { return 32 * waves_for(d) / slices_for(d); }
 constexpr int kXcds = 8;
 
 struct PrefillParams {
@@ -1542,29 +1534,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restr
   }
 }
 
-constexpr int kCus = 256;       // MI355X compute units
-constexpr int kMaxSplits = 64;
-
-size_t prefill_workspace(int splits, int count, int q_heads, int head_dim) {
-  if (splits <= 1) return 0;
-  const size_t pairs = (size_t)count * q_heads;
-  // Partial outputs, then the (max, sum) pairs, each 256-byte aligned.
-  const size_t o_bytes = ((size_t)splits * pairs * head_dim * 4 + 255) & ~(size_t)255;
-  return o_bytes + (((size_t)splits * pairs * 8 + 255) & ~(size_t)255);
-}
-
 using pda_internal::fail;
 using pda_internal::ok;
-
-// The kernel width serving a head dim: the head dim itself when a kernel
-// has it, else the next wider one (GEN kernels; odd head dims the odd
-// kernels); 0 for head dims the library does not serve (above 512).
-int prefill_dim(int head_dim) {
-  if (head_dim < 1 || head_dim > 512) return 0;
-  for (int d : {64, 96, 128, 256, 512})
-    if (head_dim <= d) return d;
-  return 0;
-}
 
 template <bool Q8, bool BF, bool GEN>
 const void* prefill_kernel_for(int kdim) {
@@ -1586,64 +1557,6 @@ const void* prefill_odd_kernel_for(int kdim) {
          : kdim == 128 ? reinterpret_cast<const void*>(paged_prefill_odd_kernel<128, Q8, BF>)
          : kdim == 256 ? reinterpret_cast<const void*>(paged_prefill_odd_kernel<256, Q8, BF>)
                        : reinterpret_cast<const void*>(paged_prefill_odd_kernel<512, Q8, BF>);
-}
-
-// How a call's work is cut.
-struct Shape {
-  bool pipe;      // the pipelined kernels
-  int blocks;     // query blocks per wave (pipelined)
-  int queries;    // per workgroup
-  int keys;       // per tile, as ranges are planned
-  int occupancy;  // workgroups per CU
-};
-
-// The pipelined kernels serve 16-bit K/V at head dims 64, 96, 128 and 256.
-// At 128 a wave may hold two blocks of queries (one wave per SIMD, half the
-// LDS reads per product): faster where the prefix is long (512 queries at
-// 32256: 228 us against 247; 4096 at 32256: 1771 against 1997), slower where
-// the chunk is short or the tiles few (512 at 0: 25 against 15 us; 1024 at
-// 4096 and 4096 at 0 level). The line is 8192 keys, and no workgroup of 256
-// queries may stay half empty (384 at 32256: 211 against 185 us).
-Shape shape_for(int head_dim, int kdim, bool q8, int start, int count, int window) {
-  const bool pipe =
-      !q8 && (head_dim == 64 || head_dim == 96 || head_dim == 128 || head_dim == 256);
-  if (!pipe)
-    return Shape{false, 1, queries_for(kdim), kdim <= 128 ? 64 : 32,
-                 kdim == 64 ? 3 : kdim <= 128 ? 2 : 1};
-  const int64_t keys = std::min<int64_t>((int64_t)start + count,
-                                         window > 0 ? (int64_t)window + count : INT64_MAX);
-  const int64_t tiles = ((int64_t)count + 127) / 128;
-  if (head_dim == 128 && keys >= 8192 && (tiles % 2 == 0 || tiles >= 8))
-    return Shape{true, 2, 256, 64, 1};
-  // (keys: the unit in which key ranges are planned, as for the other kernels.)
-  return Shape{true, 1, 128, head_dim == 256 ? 32 : 64, head_dim == 64 ? 3 : head_dim == 256 ? 1 : 2};
-}
-
-// Key ranges per (query tile, head): 1 when the tiles and heads alone give
-// every workgroup slot of the GPU (CUs x the kernel's occupancy) its work,
-// else as many as fit the slots in one round: the ranges of a chunk over a
-// long prefix are all alike, so a partly filled second round would cost a
-// whole range's time. One exception: a causal chunk that fills at most one
-// round and whose first query tile sees at most half the keys of its last
-// (a prompt from position 0) takes 2 ranges, so that the halves of its
-// longest tiles run beside its short ones. Each range holds at least 8 key
-// tiles. `request` > 0 forces a count.
-int prefill_splits(int start, int count, int q_heads, const Shape& sh, int window, int request) {
-  if (request > 0) return request < kMaxSplits ? request : kMaxSplits;
-  const int queries = sh.queries;
-  const int64_t wgs = (int64_t)(count + queries - 1) / queries * q_heads;
-  const int64_t slots = (int64_t)kCus * sh.occupancy;
-  const int keys = sh.keys;
-  // Keys seen by the chunk's first and last query tiles.
-  const int64_t cap = window > 0 ? (int64_t)window + queries : INT64_MAX;
-  const int64_t first = std::min<int64_t>((int64_t)start + std::min(count, queries), cap);
-  const int64_t span = std::min<int64_t>((int64_t)start + count, cap);
-  const int64_t by_keys = (span + keys - 1) / keys / 8;
-  if (wgs * 2 > slots) return wgs <= slots && 2 * first <= span && by_keys >= 2 ? 2 : 1;
-  int64_t s = slots / wgs;
-  if (s > by_keys) s = by_keys;
-  if (s > kMaxSplits) s = kMaxSplits;
-  return s < 1 ? 1 : (int)s;
 }
 
 template <bool BF>
@@ -1722,12 +1635,13 @@ int prefill(const void* queries, const void* keys, const void* values, const voi
   if (q8 && (((uintptr_t)key_scales | (uintptr_t)value_scales) & 1))
     return fail(PDA_ERR_ALIGNMENT, "fp16 scale arenas must be 2-byte aligned");
   if ((uintptr_t)table & 3) return fail(PDA_ERR_ALIGNMENT, "the table must be 4-byte aligned");
-  const Shape sh = shape_for(head_dim, kdim, q8, start, count, window);
-  const int nsplit = prefill_splits(start, count, q_heads, sh, window, splits);
-  const int per_wg = sh.queries;
-  // (Counted in the narrowest workgroups, whichever run.)
-  const int narrow = queries_for(kdim);
-  if ((int64_t)((count + (int64_t)narrow - 1) / narrow) * q_heads * nsplit > INT32_MAX)
+  const bool pipe = pipelined(head_dim, q8);
+  const int nsplit = prefill_splits(start, count, q_heads, kdim, window, splits);
+  const int blocks =
+      pipe ? query_blocks(start, count, q_heads, head_dim, window, softcap, nsplit) : 1;
+  const int per_wg = blocks * queries_for(kdim);
+  // (Counted with one query block a wave, whichever run.)
+  if (((int64_t)count + queries_for(kdim) - 1) / queries_for(kdim) * q_heads * nsplit > INT32_MAX)
     return fail(PDA_ERR_INVALID_ARGUMENT, "query tiles x query heads x splits exceeds 2^31");
   const size_t need = prefill_workspace(nsplit, count, q_heads, kdim);
   if (need > 0 && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)))
@@ -1770,7 +1684,7 @@ int prefill(const void* queries, const void* keys, const void* values, const voi
   prm.count = count;
   prm.tiles = (count + per_wg - 1) / per_wg;
   prm.splits = nsplit;
-  const int tile_keys = sh.keys;
+  const int tile_keys = kdim <= 128 ? 64 : 32;
   prm.page_step = tile_keys % page_size == 0 ? tile_keys / page_size : 0;
   prm.hq = q_heads;
   prm.hkv = kv_heads;
@@ -1782,13 +1696,14 @@ int prefill(const void* queries, const void* keys, const void* values, const voi
   prm.cap_in = softcap > 0.0f ? 2.0f * kLog2e * scale / softcap : 0.0f;
   prm.cap_out = softcap * kLog2e;
   void* args[] = {&prm};
-  const void* fn = sh.pipe ? (bf16_elems ? pipe_kernel_for<true>(kdim, sh.blocks) : pipe_kernel_for<false>(kdim, sh.blocks))
+  const void* fn = pipe ? (bf16_elems ? pipe_kernel_for<true>(kdim, blocks)
+                                      : pipe_kernel_for<false>(kdim, blocks))
                   : q8 ? prefill_kernel_for<true, false>(kdim, gen, odd)
                   : bf16_elems ? prefill_kernel_for<false, true>(kdim, gen, odd)
                                : prefill_kernel_for<false, false>(kdim, gen, odd);
   const hipStream_t hs = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)((int64_t)prm.tiles * q_heads * nsplit));
-  hipError_t err = hipLaunchKernel(fn, grid, dim3(sh.pipe ? 256 : 64 * waves_for(kdim)), args, 0, hs);
+  hipError_t err = hipLaunchKernel(fn, grid, dim3(64 * waves_for(kdim)), args, 0, hs);
   if (err != hipSuccess)
     return fail(PDA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(err));
   if (nsplit > 1) {
@@ -1823,14 +1738,9 @@ int pda_prefill_workspace_bytes(int32_t start, int32_t count, int32_t q_heads,
   const int kdim = prefill_dim(head_dim);
   if (kdim == 0)
     return fail(PDA_ERR_HEAD_DIM, "head_dim %d: prefill serves head dims 1..512", head_dim);
-  // The same bytes for 16-bit and 8-bit caches, whose kernels differ.
-  int s = 1;
-  *bytes = 0;
-  for (int q8 = 1; q8 >= 0 && count > 0; --q8) {
-    s = prefill_splits(start, count, q_heads, shape_for(head_dim, kdim, q8, start, count, window), window, splits);
-    *bytes = std::max(*bytes, prefill_workspace(s, count, q_heads, kdim));
-  }
+  const int s = count == 0 ? 1 : prefill_splits(start, count, q_heads, kdim, window, splits);
   if (splits_used) *splits_used = s;
+  *bytes = prefill_workspace(s, count, q_heads, kdim);
   return ok();
 }
 

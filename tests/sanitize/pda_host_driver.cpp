@@ -87,8 +87,8 @@ void planner_sweep() {
 }
 
 void prefill_planner_sweep() {
-  const int32_t starts[] = {0, 1, 500, 4096, 1 << 20, 2147483647 - 600, -1};
-  const int32_t counts[] = {0, 1, 100, 512, 4096, 1 << 16, -1};
+  const int32_t starts[] = {0, 1, 500, 4096, 32256, 1 << 20, 2147483647 - 600, -1};
+  const int32_t counts[] = {0, 1, 100, 512, 1152, 4096, 1 << 16, -1};
   const int32_t heads[] = {1, 8, 28, 128, 0};
   const int32_t dims[] = {2, 4, 64, 80, 96, 128, 130, 256, 510, 512, 0, 1, 514};
   const int32_t windows[] = {0, 1, 256, -1};

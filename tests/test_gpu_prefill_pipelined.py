@@ -93,3 +93,52 @@ def test_moving_max(gpu, d, start):
     q, k, v, table = c["t"]
     c["t"] = (q, torch.as_tensor(c["keys"], device=gpu), v, table)
     check(c, scale=4 * d ** -0.5, what=f"D{d} moving max @{start}")
+
+
+# Calls whose two-block workgroups fill the CUs as well as one-block ones do
+# (q heads, count, start, page, window, splits, images), all of one kv head.
+TWO_BLOCKS = [
+    (64, 256, 7936, 16, 0, 0, ()),               # at the line, whole workgroups
+    (64, 255, 7937, 24, 0, 4, ()),               # the last wave one query short
+    (64, 193, 8001, 16, 0, 0, ()),               # the second half of 256 a wave and a query
+    (16, 1000, 7300, 64, 8300, 0, ()),           # ragged, a window over all keys
+    (16, 993, 7300, 5, 0, 8, ((7200, 300), (8100, 150))),
+]
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("hq,count,start,page,window,splits,images", TWO_BLOCKS)
+def test_two_blocks_that_fill_the_cus(gpu, bf16, hq, count, start, page, window, splits, images):
+    from instinct_amd.hip_kernels import paged_prefill_attention
+
+    gen = torch.Generator(device=gpu).manual_seed(count)
+    dtype = torch.bfloat16 if bf16 else torch.float16
+    keys = start + count
+    pages = -(-keys // page)
+    table = torch.randperm(pages + 3, generator=gen, device=gpu)[:pages].int()
+    draw = lambda *shape: torch.randn(shape, generator=gen, device=gpu).to(dtype)  # noqa: E731
+    q, k, v = draw(count, hq, 128), draw(pages + 3, 1, page, 128), draw(pages + 3, 1, page, 128)
+    scale = 128 ** -0.5
+    if count == 193:  # scores that keep growing: the outputs are rescaled many times
+        ramp = torch.linspace(0.05, 3.0, pages * page, device=gpu).view(pages, 1, page, 1)
+        k[table.long()] = (k[table.long()] * ramp).to(dtype)
+        scale *= 4
+    released = pages // 2
+    table[released] = -1
+    got = paged_prefill_attention(q, k, v, table, start=start, page_size=page, scale=scale,
+                                  window=window, splits=splits, images=images)
+    rows = [t[table.long().clamp(min=0), 0].reshape(-1, 128)[:keys].double() for t in (k, v)]
+    pos = start + torch.arange(count, device=gpu)[:, None]
+    key = torch.arange(keys, device=gpu)[None, :]
+    seen = key <= pos
+    for at, length in images:
+        seen |= (pos >= at) & (pos < at + length) & (key >= at) & (key < at + length)
+    seen &= (key // page) != released
+    worst = total = 0.0
+    for h in range(hq):
+        s = torch.matmul(q[:, h].double(), rows[0].t().contiguous()) * scale
+        want = torch.matmul(torch.softmax(s.masked_fill(~seen, -torch.inf), -1), rows[1])
+        diff = (got[:, h].double() - want).abs()
+        worst, total = max(worst, diff.max().item()), total + diff.mean().item() / hq
+    # The bars of the other prefill tests (fp16; bf16: 8 times, the formats' ratio).
+    assert worst <= 2e-3 * (8 if bf16 else 1) and total <= 2e-4 * (8 if bf16 else 1)
