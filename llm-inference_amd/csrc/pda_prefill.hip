@@ -1466,7 +1466,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
 }
 
 template <int D, int QB, bool BF>
-__global__ __launch_bounds__(256, D * QB <= 128 ? 2 : 1) void paged_prefill_pipe_kernel(
+__global__ __launch_bounds__(256, QB == 1 ? occupancy_for(D) : 1) void paged_prefill_pipe_kernel(
     const PrefillParams p) {
   prefill_pipe_body<D, QB, BF>(p);
 }

@@ -21,7 +21,8 @@ constexpr int slices_for(int d) { return d > 256 ? 4 : 1; }
 constexpr int waves_for(int d) { return d > 256 ? 2 * kWaves : kWaves; }
 // Queries per workgroup: 32 per query block.
 constexpr int queries_for(int d) { return 32 * waves_for(d) / slices_for(d); }
-// Workgroups per CU that the key ranges are planned for.
+// Workgroups per CU that the key ranges are planned for. The pipelined
+// kernels' launch bounds hold them to it (with one query block a wave).
 constexpr int occupancy_for(int d) { return d == 64 ? 3 : d <= 128 ? 2 : 1; }
 
 constexpr int kCus = 256;  // MI355X compute units
