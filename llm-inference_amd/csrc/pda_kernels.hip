@@ -355,8 +355,8 @@ constexpr int64_t kLocalMaxUnits = 512;
 constexpr int64_t kLocalMaxUnitBytes = int64_t(3) << 19;  // 1.5 MiB
 constexpr size_t kLocalMaxLds = size_t(64) << 10;
 
-size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, int page_size,
-                 int waves, int ring, int grid_groups) {
+size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, bool gen,
+                 int page_size, int waves, int ring, int grid_groups) {
   const int grid_pairs = grid_groups * (waves / 2);
   const size_t lds = (size_t)pda_decode::local_lds_offset(batch) * sizeof(int32_t) +
                      (size_t)waves * pl.unit_heads * (dim * sizeof(float) + sizeof(float2));
@@ -383,20 +383,43 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, int
   // one page at a time) 28/4 of 128, 1 x 256 11.5 / 12.8, 1 x 384 13.7 / 13.1,
   // 16 x 512 16.3 / 17.7, 16 x 768 20.0 / 17.9; one head a unit, 32/32 of 80,
   // 1 x 384 10.3 / 11.5, 1 x 768 14.0 / 12.0, 4 x 768 15.0 / 17.2; 8/4 of 256,
-  // 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0. Units past the resident
-  // workgroups keep the rule above.
+  // 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0.
   const int64_t unit_keys = pl.unit_pages_max * page_size;
   const bool many = units >= 64;
-  const int64_t short_keys = dim > 128              ? 256
-                             : dim <= 64            ? (many ? 768 : 512)
-                             : pl.mf                ? (many ? 512 : 320)
-                             : pl.unit_heads == 1   ? (many ? 768 : 384)
-                                                    : (many || dim < 128 ? 768 : 640);
+  int64_t short_keys = dim > 128              ? 256
+                       : dim <= 64            ? (many ? 768 : 512)
+                       : pl.mf                ? (many ? 512 : 320)
+                       : pl.unit_heads == 1   ? (many ? 768 : 384)
+                                              : (many || dim < 128 ? 768 : 640);
+  // The generic kernels take a wave two to four times as long per key above 64
+  // dims, so their lines lie lower: a unit of one head (or few enough units to be
+  // cut into heads) by what the stream has to merge, others by what they leave
+  // idle. Local / stream: 24/8 heads of 112, 1 x 256 keys 13.5 / 16.3, 1 x 384
+  // 17.2 / 16.6, 16 x 128 14.8 / 16.8, 16 x 256 21.6 / 18.3, 16 x 768 49.4 / 28.5,
+  // at 8 bits 16 x 384 21.8 / 23.1, 16 x 512 26.1 / 24.5; 32/8 of 96 at 8 bits, 1
+  // x 384 15.1 / 18.0, 1 x 512 17.7 / 18.1; 16/4, 64 x 768 31.9 / 36.4; 16/16 of
+  // 72, 4 x 512 16.1 / 14.8, 16 x 768 21.2 / 27.2; 32/32 of 80 at 8 bits, 4 x 512
+  // 17.6 / 18.4, 4 x 768 22.9 / 21.5; 8/8 of 160, 1 x 128 12.2 / 15.1, 1 x 256
+  // 17.7 / 15.6; 8/2 of 200, 16 x 256 at 8 bits 18.7 / 20.5, 64 x 64 13.9 / 19.2,
+  // 64 x 256 31.6 / 22.2.
+  if (gen && dim > 64) {
+    const int64_t single = units * pl.unit_heads;
+    const bool cut = single <= 256;  // CUs
+    if (dim > 128)
+      short_keys = !cut ? 64 : pl.unit_heads > 1 ? 256 : 192;
+    else if (!cut)
+      short_keys = std::min<int64_t>((elem == 1 ? 3 : 1) * units, 768);
+    else
+      short_keys = std::max<int64_t>(elem == 1 && pl.unit_heads > 1 ? 448 : 320,
+                                     std::min<int64_t>((elem == 1 ? 4 : 3) * single, 768));
+  }
   if (units <= grid_groups && unit_keys <= short_keys) return lds;
   // More units than resident workgroups, of several heads: the stream's even
   // split wins back its second launch (32/8 heads, 64 sequences of 256 keys,
   // stream / local: 23.1 / 25.7 at head dim 128, 24.7 / 31.8 at 96, 20.1 / 21.7
-  // at 8 bits; of 64 keys level; two heads of 256 level).
+  // at 8 bits). Units of up to a page a wave keep the rule below (64 sequences
+  // of 64 keys: 15.8 / 15.3 at 128 and 8 bits, 17.2 / 17.3 at 16, 20.0 / 14.4 at
+  // 96 and 8 bits, but 19.0 / 22.4 at 16; 16/8 heads of 256 14.9 / 17.2).
   if (units > grid_groups && pl.unit_heads > 2 && pl.unit_pages_max > waves) return 0;
   return units <= kLocalMaxUnits && unit_bytes <= kLocalMaxUnitBytes && short_waves ? lds : 0;
 }
@@ -527,7 +550,7 @@ int plan_launch(Plan& pl, int32_t batch, int32_t kv_heads, int32_t head_dim,
   }
   const int grid_pairs = lp.groups * (lp.kp.split_waves / 2);
   lp.dim = pl.mf ? head_dim : kernel_dim(head_dim, q8);
-  lp.lds_local = local_lds(pl, batch, kv_heads, lp.dim, q8 ? 1 : 2, page_size,
+  lp.lds_local = local_lds(pl, batch, kv_heads, lp.dim, q8 ? 1 : 2, lp.kp.gen, page_size,
                            lp.kp.split_waves, lp.kp.ring, lp.groups);
   // Local mode on the VALU kernels, when a unit per GQA group leaves CUs
   // idle: a unit per query head, as long as the units still fit one
