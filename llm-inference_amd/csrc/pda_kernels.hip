@@ -210,6 +210,7 @@ struct Plan {
   int min_pages = 0;
   int64_t pages_est = 0;       // visible pages of the batch if every length = longest
   int64_t unit_pages_max = 0;  // visible pages of one unit, at most
+  int64_t unit_keys_max = 0;   // and its visible keys
   size_t off_meet = 0, off_ml = 0, off_o = 0, total = 0;
 };
 
@@ -257,6 +258,9 @@ int make_plan(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t head_dim
   int64_t est = pages_max;
   if (longest > 0) est = std::min<int64_t>(est, (longest + page_size - 1) / page_size + 1);
   pl.unit_pages_max = est;
+  pl.unit_keys_max = (int64_t)table_stride * page_size;
+  if (longest > 0) pl.unit_keys_max = std::min<int64_t>(pl.unit_keys_max, longest);
+  if (window > 0) pl.unit_keys_max = std::min<int64_t>(pl.unit_keys_max, window);
   pl.pages_est = (int64_t)batch * kv_heads * pl.nhg * est;
   pl.min_pages = split_pages > 0 ? split_pages : kMinPagesPerWave;
   // Workspace: the per-sequence page prefix, the meeting points of the wave
@@ -383,8 +387,9 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, boo
   // one page at a time) 28/4 of 128, 1 x 256 11.5 / 12.8, 1 x 384 13.7 / 13.1,
   // 16 x 512 16.3 / 17.7, 16 x 768 20.0 / 17.9; one head a unit, 32/32 of 80,
   // 1 x 384 10.3 / 11.5, 1 x 768 14.0 / 12.0, 4 x 768 15.0 / 17.2; 8/4 of 256,
-  // 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0.
-  const int64_t unit_keys = pl.unit_pages_max * page_size;
+  // 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0. Counted in visible keys: the
+  // same call over a wider table or larger pages takes the same side (64 x 768
+  // keys, 14/2 heads of 64, a table of 256 pages: local / stream 14.4 / 18.5).
   const bool many = units >= 64;
   int64_t short_keys = dim > 128              ? 256
                        : dim <= 64            ? (many ? 768 : 512)
@@ -413,7 +418,7 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, boo
       short_keys = std::max<int64_t>(elem == 1 && pl.unit_heads > 1 ? 448 : 320,
                                      std::min<int64_t>((elem == 1 ? 4 : 3) * single, 768));
   }
-  if (units <= grid_groups && unit_keys <= short_keys) return lds;
+  if (units <= grid_groups && pl.unit_keys_max <= short_keys) return lds;
   // More units than resident workgroups, of several heads: the stream's even
   // split wins back its second launch (32/8 heads, 64 sequences of 256 keys,
   // stream / local: 23.1 / 25.7 at head dim 128, 24.7 / 31.8 at 96, 20.1 / 21.7

@@ -57,6 +57,17 @@ def test_rules(hq, hkv, d, batch, longest, kind, local, merge):
     assert choice(hq, hkv, d, batch, longest, kind) == (local, merge)
 
 
+@pytest.mark.parametrize("hq,hkv,d,batch,longest,kind,local,merge", LINES)
+def test_rules_over_wider_tables(hq, hkv, d, batch, longest, kind, local, merge):
+    """The lines count visible keys: a call at a line stays on its side over a
+    wider table, with larger pages, or where a window and not the length ends
+    the keys."""
+    if local:
+        assert choice(hq, hkv, d, batch, longest, kind, width=200)[0] == 1
+        assert choice(hq, hkv, d, batch, longest, kind, page=64, width=64)[0] == 1
+        assert choice(hq, hkv, d, batch, 4096, kind, width=256, window=longest)[0] == 1
+
+
 def arena(gpu, gen, kind, layout, pages, hkv, d):
     """K or V of one call: the arena, its scales, and its rows in float64."""
     shape = (pages, hkv, PAGE, d)
