@@ -368,9 +368,11 @@ def prefill_leg(w, tokens, steps, start=0):
     tflops = flops / (med * 1e-3) / 1e12
     bf16 = dtype == torch.bfloat16
     width = next(x for x in (64, 96, 128, 256, 512) if d <= x)  # the kernel that serves d
-    return {"kernel": f"paged_prefill_kernel<{width},false,{str(bf16).lower()},"
-                      f"{str(width != d).lower()}> "
-                      f"(pda_paged_prefill_attention{'_bf16' if bf16 else ''})",
+    # 16-bit K/V of the narrower widths: the pipelined kernels <D, query blocks, BF>.
+    name = (f"paged_prefill_pipe_kernel<{d},{'1|2' if d == 128 else 1},{str(bf16).lower()}>"
+            if d in (64, 96, 128, 256) else
+            f"paged_prefill_kernel<{width},false,{str(bf16).lower()},{str(width != d).lower()}>")
+    return {"kernel": f"{name} (pda_paged_prefill_attention{'_bf16' if bf16 else ''})",
             "tokens": tokens, "start": start, "key_ranges": splits, "q_heads": hq,
             "kv_heads": hkv, "head_dim": d,
             "us_median": round(med * 1e3, 2), "flops": flops,

@@ -383,13 +383,15 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, boo
   // higher from 64 units on, where the stream has more to merge. Local /
   // stream, us a call among others: 14/2 heads of 64, 1 x 384 keys 10.1 / 10.9,
   // 1 x 768 13.5 / 11.0, 64 x 512 12.5 / 19.1; 32/8 of 128, 1 x 512 11.4 / 13.5,
-  // 1 x 768 14.2 / 13.6, 16 x 768 19.7 / 20.3; of 96, 1 x 768 14.6 / 17.3; on the matrix cores (a wave takes
-  // one page at a time) 28/4 of 128, 1 x 256 11.5 / 12.8, 1 x 384 13.7 / 13.1,
-  // 16 x 512 16.3 / 17.7, 16 x 768 20.0 / 17.9; one head a unit, 32/32 of 80,
-  // 1 x 384 10.3 / 11.5, 1 x 768 14.0 / 12.0, 4 x 768 15.0 / 17.2; 8/4 of 256,
-  // 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0. Counted in visible keys: the
-  // same call over a wider table or larger pages takes the same side (64 x 768
-  // keys, 14/2 heads of 64, a table of 256 pages: local / stream 14.4 / 18.5).
+  // 1 x 768 14.2 / 13.6, 16 x 768 19.7 / 20.3; of 96, 1 x 768 14.6 / 17.3; on
+  // the matrix cores (a wave takes one page at a time) 28/4 of 128, 1 x 256 11.5
+  // / 12.8, 1 x 384 13.7 / 13.1, 16 x 512 16.3 / 17.7, 16 x 768 20.0 / 17.9; one
+  // head a unit, 32/32 of 80, 1 x 384 10.3 / 11.5, 1 x 768 14.0 / 12.0, 4 x 768
+  // 15.0 / 17.2; 8/4 of 256, 1 x 256 11.0 / 12.8, 1 x 384 13.5 / 13.0. (Not the
+  // last word from 64 units on: 14/2 heads of 64, 64 x 1024 16.5 / 19.3; 16/16,
+  // 16 x 1024 15.5 / 18.0.) Counted in visible keys: the same call over a wider
+  // table or larger pages takes the same side (64 x 768 keys, 14/2 heads of 64,
+  // a table of 256 pages: 14.4 / 18.5).
   const bool many = units >= 64;
   int64_t short_keys = dim > 128              ? 256
                        : dim <= 64            ? (many ? 768 : 512)

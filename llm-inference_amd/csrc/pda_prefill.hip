@@ -866,38 +866,40 @@ __device__ __forceinline__ void prefill_body(const PrefillParams p) {
 // The pipelined kernels: 16-bit K/V at head dims 64, 96, 128 and 256.
 //
 // The tile loop of prefill_body computes S, softmax and P V of a tile one
-// after the other and moves K/V through registers on its way into LDS; a wave
-// spent 5,000 - 6,000 cycles on a 64-key tile at D = 128 that holds 1,024
-// cycles of matrix-core work, spread over every phase. Here
+// after the other and moves K/V through registers on its way into LDS; the
+// matrix cores were busy 31-34% of its cycles at D = 128. Here
 //  * a step interleaves, instruction by instruction, the products of one
 //    32-key block's V, the scores of a later block and the weights of the
 //    block between them, so that one wave alone keeps the matrix core busy
 //    while its exps run (`step`);
 //  * K and V go from global memory straight into LDS (copies spread over the
-//    slots of a step: issued together they stalled a wave for 1,250 cycles a
-//    tile), in planes of 64 bytes per key whose reads touch each bank once:
-//    V as it lies, K with its 16-byte chunks permuted by key;
+//    slots of a step), in planes of 64 bytes per key whose reads touch each
+//    bank once: V as it lies, K with its 16-byte chunks permuted by key;
 //  * V runs one tile behind K, so that two LDS tiles of each serve the
 //    pipeline with one barrier per tile;
 //  * what only some tiles need (masks, softcap, the running max) sits behind
 //    one wave-uniform test per step.
-// What bounds it: at D = 128 with one query block a wave (two workgroups per
-// CU) a step takes 1,040 - 1,320 cycles for 1,024 of the two waves'
-// matrix-core work, and the power limit (2.0 GHz under this load, 2.3 GHz
-// with two blocks a wave, which read K and V from LDS half as often). 4096
-// tokens at 0, 28/4 heads: 158 -> 141 us; 512 at 32256: 279 -> 228 us; 4096 at
-// 32256 1.14 PFLOP/s. D = 64 (14/2 heads, 1531 at 389): 30.8 -> 26.0 us. D = 256
-// (16/8 heads, 2048 at 6144, window 1024): 80 -> 59 us.
+// What bounds it (counters): at D = 128 with one query block a wave (4096
+// tokens at 0, 28/4 heads) the matrix cores are busy 39% of the cycles, the VALU
+// 36% (6.4 of its instructions a product), no LDS bank conflicts, 38% of the
+// waves' cycles waiting; with two blocks, which read K and V from LDS half as
+// often (512 at 32256), 42%, 33% (5.4) and 27%. At D = 256 (16/8 heads, 2048 at
+// 6144, window 1024) 23% and 16%: one wave per SIMD, masks and short ranges; at D =
+// 64 (14/2 heads, 1531 at 389) 10% and 21%: 15 VALU instructions a product, a
+// launch of a few tiles a workgroup.
+// us a call, prefill_body / here: 4096 at 0 158 / 141; 512 at 32256, bf16, 279 /
+// 227; 4096 at 32256 2220 / 1795; D = 64, 1531 at 389 30.8 / 26.0; D = 256,
+// 2048 at 6144, window 1024 80 / 57.
 //
 // Short calls: the queries' loads, the table entries and the first tiles' copies
 // are under way together, a 32-key block past a wave's last key is left out, and
 // outputs that are still zeros are not rescaled. 16/8 heads of 256, 19 tokens at
 // 0: 6.8 us; 9.6 with the loads in a row, both blocks always and the rescaling.
 //
-// Measured and not kept: the weights' sum on v_dot2 inside the step (each
-// holds the matrix pipe for 18 cycles: step 1,156 against 1,040), fp32 adds
-// of the rounded weights instead (level), operands read 2, 4 or 5 ahead
-// instead of 3 (level), two query blocks a wave at D = 64 (31.7 us).
+// Measured and not kept: the weights' sum on v_dot2 inside the step (it holds
+// the matrix pipe; slower), fp32 adds of the rounded weights instead (level),
+// operands read 2, 4 or 5 ahead instead of 3 (level), two query blocks a wave at
+// D = 64 (31.7 us).
 //
 // QB: blocks of 32 queries per wave.
 template <int D, int QB, bool BF>
@@ -927,7 +929,10 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
     const int j = item / kXcds;
     // Where the XCDs hold several query tiles at once (fewer than 8 kv
     // heads), every other round hands them out in reverse, so that no XCD
-    // gets the longer tile each time.
+    // gets the longer tile each time (us, in one direction / reversed: 28/4
+    // heads of 128, 4096 tokens at 0 147.0 / 143.3; 14/2, 8192 at 0 278 / 255;
+    // 14/2 of 64, 4096 at 0 60.7 / 59.2; where tiles are alike 0.2-0.4 us the
+    // other way: 512 at 2048, 28/4 of 128 37.0 / 37.2).
     if ((j / G) & 1 && kXcds % p.hkv == 0) x = kXcds - p.hkv - x / p.hkv * p.hkv + x % p.hkv;
     item = ((j / G) * kXcds + x) * G + j % G;
   }
@@ -1000,10 +1005,11 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
   const int vchunk = 8 * (lane & 3);
   const uint32_t k_dst = uniform(lds_address(&s_k[0][0]) + 1024 * w);
   const uint32_t v_dst = uniform(lds_address(&s_v[0][0]) + 1024 * w);
-  // The page of this thread's key is looked up two iterations before its rows
-  // are copied, so nothing waits for it; each wave looks up the pages of all
-  // 64 keys of the tile as well (one per lane) for the mask of usable keys,
-  // which then needs neither LDS nor a barrier.
+  // The page of this thread's key is looked up one iteration before its rows
+  // are copied (its K's; two for V's): the wait is that iteration's own, at its
+  // end, with its copies'. Each wave looks up the pages of all 64 keys of the
+  // tile as well (one per lane) for the mask of usable keys, which then needs
+  // neither LDS nor a barrier.
   const uint32_t pages = (uint32_t)min(p.arena_pages, (int64_t)INT32_MAX);
   const uint32_t step_pages = kKeys / page_size, step_rows = kKeys % page_size;
   int page = 0, row_off = 0, page_m = 0;
@@ -1111,7 +1117,7 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
       // not past its position, inside its window, or inside its image. Two
       // instructions per score then (bit to mask, select), where a test of
       // each key's position took nine: the diagonal tiles are most of a short
-      // prompt (4096 tokens: 12 of the 117 us of its longest workgroup).
+      // prompt.
       const int hi = qpos + 32 * j - k0;
       uint32_t see = below(hi + 1);
       if (p.window > 0) see &= ~below(hi - p.window + 1);
@@ -1136,8 +1142,8 @@ __device__ __forceinline__ void prefill_pipe_body(const PrefillParams p) {
     pb[i / 4][2 * (i % 4)] = ph[0];
     pb[i / 4][2 * (i % 4) + 1] = ph[1];
   };
-  // Their sum, all of a block's at once: v_dot2 holds the matrix pipe, and
-  // one between two matrix-core instructions costs 18 cycles of it.
+  // Their sum, all of a block's at once: v_dot2 holds the matrix pipe, so none
+  // goes between two products.
   auto total = [&](const f16x8 (&pb)[2], float sum) {
     float s2[2] = {sum, 0.0f};
 #pragma unroll
