@@ -359,7 +359,9 @@ constexpr int64_t kLocalMaxUnits = 512;
 constexpr int64_t kLocalMaxUnitBytes = int64_t(3) << 19;  // 1.5 MiB
 constexpr size_t kLocalMaxLds = size_t(64) << 10;
 
-size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, bool gen,
+// `fit`: the generic kernels' own lines do not count (a call whose stream mode
+// does not fit the static scratch).
+size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, bool gen, bool fit,
                  int page_size, int waves, int ring, int grid_groups) {
   const int grid_pairs = grid_groups * (waves / 2);
   const size_t lds = (size_t)pda_decode::local_lds_offset(batch) * sizeof(int32_t) +
@@ -409,7 +411,7 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, boo
   // 17.6 / 18.4, 4 x 768 22.9 / 21.5; 8/8 of 160, 1 x 128 12.2 / 15.1, 1 x 256
   // 17.7 / 15.6; 8/2 of 200, 16 x 256 at 8 bits 18.7 / 20.5, 64 x 64 13.9 / 19.2,
   // 64 x 256 31.6 / 22.2.
-  if (gen && dim > 64) {
+  if (gen && dim > 64 && !fit) {
     const int64_t single = units * pl.unit_heads;
     const bool cut = single <= 256;  // CUs
     if (dim > 128)
@@ -542,7 +544,8 @@ struct LaunchPlan {
 };
 
 int plan_launch(Plan& pl, int32_t batch, int32_t kv_heads, int32_t head_dim,
-                int32_t page_size, bool q8, bool bf16, bool need_device, LaunchPlan* out) {
+                int32_t page_size, bool q8, bool bf16, bool need_device, LaunchPlan* out,
+                bool fit = false) {
   LaunchPlan lp;
   lp.kp = pl.mf ? (head_dim == 512 ? kernels_mf512(q8, bf16)
                    : q8 ? (bf16 ? kernels_mf_q8_bf16(head_dim) : kernels_mf_q8(head_dim))
@@ -557,7 +560,7 @@ int plan_launch(Plan& pl, int32_t batch, int32_t kv_heads, int32_t head_dim,
   }
   const int grid_pairs = lp.groups * (lp.kp.split_waves / 2);
   lp.dim = pl.mf ? head_dim : kernel_dim(head_dim, q8);
-  lp.lds_local = local_lds(pl, batch, kv_heads, lp.dim, q8 ? 1 : 2, lp.kp.gen, page_size,
+  lp.lds_local = local_lds(pl, batch, kv_heads, lp.dim, q8 ? 1 : 2, lp.kp.gen, fit, page_size,
                            lp.kp.split_waves, lp.kp.ring, lp.groups);
   // Local mode on the VALU kernels, when a unit per GQA group leaves CUs
   // idle: a unit per query head, as long as the units still fit one
@@ -640,9 +643,22 @@ int decode(int passes, const void* queries, const void* keys, const void* values
       return fail(PDA_ERR_ALIGNMENT, "workspace must be 256-byte aligned");
   }
 
+  const Plan asked = pl;
   LaunchPlan lp;
   rc = plan_launch(pl, batch, kv_heads, head_dim, page_size, q8, bf16, true, &lp);
   if (rc) return rc;
+  auto scratch_layout = [&] {
+    return workspace_layout(batch, pl.unit_heads, kernel_dim(head_dim, q8),
+                            (int64_t)lp.groups * (lp.kp.split_waves / 2),
+                            (int64_t)lp.groups * 2 * lp.kp.split_waves);
+  };
+  // Short units of the generic kernels fit the scratch in local mode, a head
+  // each, where their stream mode does not: slower is better than refused.
+  if (use_scratch && !lp.lds_local && scratch_layout().total > kScratchBytes) {
+    pl = asked;
+    rc = plan_launch(pl, batch, kv_heads, head_dim, page_size, q8, bf16, true, &lp, true);
+    if (rc) return rc;
+  }
   const KernelPair& kp = lp.kp;
   const size_t lds = lp.lds;
   const int wg_pairs = kp.split_waves / 2;
@@ -657,8 +673,7 @@ int decode(int passes, const void* queries, const void* keys, const void* values
   wl.off_o = pl.off_o;
   wl.total = pl.total;
   if (use_scratch) {
-    wl = workspace_layout(batch, pl.unit_heads, kernel_dim(head_dim, q8), (int64_t)groups * wg_pairs,
-                          (int64_t)groups * 4 * wg_pairs);
+    wl = scratch_layout();
     if (wl.total > kScratchBytes)
       return fail(PDA_ERR_WORKSPACE,
                   "the no-allocation call needs %zu bytes of scratch for this shape, above "

@@ -103,3 +103,16 @@ def test_noalloc_rejects_a_shape_beyond_its_scratch(gpu):
     assert "no-allocation" in _lib.library().pda_last_error().decode()
     # The same call with a workspace works.
     within_bar(with_workspace(w, False), oracle(w), "512-wide with a workspace")
+
+
+@pytest.mark.parametrize("hq,hkv,d,lengths", [
+    (64, 8, 112, [500]), (64, 8, 112, [1, 640, 300, 17]), (8, 2, 200, [250] * 40),
+    (64, 8, 72, [600, 64])])
+def test_noalloc_takes_short_units_of_the_generic_kernels(gpu, hq, hkv, d, lengths):
+    """Eight (four) heads a unit at padded widths of 128 (256): the stream's
+    partials would not fit the scratch where two workgroups a CU are resident,
+    local mode's, a head a unit, do."""
+    w = workloads.reference_test_case(hq, hkv, d, lengths, 0, 0.0, device=gpu)
+    rc, got = noalloc(w, 0)
+    _lib.check(rc)
+    within_bar(got, oracle(w), f"{hq}/{hkv} heads of {d}, {lengths}")
