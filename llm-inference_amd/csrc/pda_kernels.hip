@@ -361,8 +361,8 @@ constexpr size_t kLocalMaxLds = size_t(64) << 10;
 
 // `fit`: the generic kernels' own lines do not count (a call whose stream mode
 // does not fit the static scratch).
-size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, bool gen, bool fit,
-                 int page_size, int waves, int ring, int grid_groups) {
+size_t local_lds(const Plan& pl, int batch, int kv_heads, int head_dim, int dim, int elem, bool gen,
+                 bool fit, int page_size, int waves, int ring, int grid_groups) {
   const int grid_pairs = grid_groups * (waves / 2);
   const size_t lds = (size_t)pda_decode::local_lds_offset(batch) * sizeof(int32_t) +
                      (size_t)waves * pl.unit_heads * (dim * sizeof(float) + sizeof(float2));
@@ -401,28 +401,45 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int dim, int elem, boo
                        : pl.unit_heads == 1   ? (many ? 768 : 384)
                                               : (many || dim < 128 ? 768 : 640);
   // The generic kernels take a wave two to four times as long per key above 64
-  // dims, so their lines lie lower: a unit of one head (or few enough units to be
-  // cut into heads) by what the stream has to merge, others by what they leave
-  // idle. Local / stream: 24/8 heads of 112, 1 x 256 keys 13.5 / 16.3, 1 x 384
-  // 17.2 / 16.6, 16 x 128 14.8 / 16.8, 16 x 256 21.6 / 18.3, 16 x 768 49.4 / 28.5,
-  // at 8 bits 16 x 384 21.8 / 23.1, 16 x 512 26.1 / 24.5; 32/8 of 96 at 8 bits, 1
-  // x 384 15.1 / 18.0, 1 x 512 17.7 / 18.1; 16/4, 64 x 768 31.9 / 36.4; 16/16 of
-  // 72, 4 x 512 16.1 / 14.8, 16 x 768 21.2 / 27.2; 32/32 of 80 at 8 bits, 4 x 512
-  // 17.6 / 18.4, 4 x 768 22.9 / 21.5; 8/8 of 160, 1 x 128 12.2 / 15.1, 1 x 256
-  // 17.7 / 15.6; 8/2 of 200, 16 x 256 at 8 bits 18.7 / 20.5, 64 x 64 13.9 / 19.2,
-  // 64 x 256 31.6 / 22.2.
+  // dims, so their lines lie lower, by how a unit's heads run: a workgroup each
+  // (the stream, whose waves take them together, is the slower the more heads),
+  // two of those to a CU, or together. Where local and stream cross, keys, 8 kv
+  // heads, 1, 2, 3, 4, 5 heads a unit; 72 / 112 / 160 / 200 dims:
+  //  1 x, 16 bits: 409 453 515 576 652 / 303 321 361 410 459 / 199 210 230 261 297
+  //    / 198 210 225 249 283; 8 bits: 365 395 459 520 585 / 364 396 468 550 619 /
+  //    175 188 232 290 335 / 173 189 240 291 330; 16 x 1 head 505-768, 24 x past
+  //    768 (384 above 128 dims);
+  //  257 to 512 heads, two to a CU: 173-485 / 410-536 at 16 / 8 bits, above 128
+  //    dims 108-224 / 146-221;
+  //  more, together: 16 x 473-614, 24 x past 768; above 128 dims 272-306, past 384.
+  // The lines follow the lower of the crossings that share them (16-bit ones by
+  // the row's length: 72 dims cross later than 112).
+  // us, local / stream: 24/8 heads of 112, 16 x 768 keys 49.4 / 28.5; 8/2 of 200,
+  // 64 x 256 31.6 / 22.2; 64/8 of 112, 1 x 341 16.6 / 23.8.
   if (gen && dim > 64 && !fit) {
-    const int64_t single = units * pl.unit_heads;
-    const bool cut = single <= 256;  // CUs
-    if (dim > 128)
-      short_keys = !cut ? 64 : pl.unit_heads > 1 ? 256 : 192;
-    else if (!cut)
-      short_keys = std::min<int64_t>((elem == 1 ? 3 : 1) * units, 768);
+    const int64_t uh = pl.unit_heads, single = units * uh;
+    const bool wide = dim > 128, bits8 = elem == 1;
+    if (single > grid_groups)
+      short_keys = (wide ? 2 : 4) * units;
+    else if (single > 256)  // CUs
+      short_keys = wide                ? (uh >= 5 && !bits8 ? 224 : bits8 ? 150 : 112)
+                   : bits8             ? (uh >= 5 ? 320 : 400)
+                   : head_dim <= 96    ? 384
+                   : uh >= 5           ? 352
+                   : uh == 2           ? 256
+                                       : 192;
     else
-      short_keys = std::max<int64_t>(elem == 1 && pl.unit_heads > 1 ? 448 : 320,
-                                     std::min<int64_t>((elem == 1 ? 4 : 3) * single, 768));
+      short_keys = std::max<int64_t>(wide    ? (bits8 ? 120 + 40 * uh : 170 + 20 * uh)
+                                     : bits8 ? (single >= 192 ? 640 : 290 + 60 * uh)
+                                             : 540 - 21 * head_dim / 8 + 40 * uh,
+                                     units >= (wide ? 192 : 128) ? 4 * units : 0);
+    short_keys = std::min<int64_t>(short_keys, wide ? 384 : 768);
   }
-  if (units <= grid_groups && pl.unit_keys_max <= short_keys) return lds;
+  // (Pages of fewer than 16 keys cost a wave what 16 do: 28/4 heads of 128, 17
+  // sequences, a window of 512 in pages of 8: 21.0 / 18.3.)
+  const int64_t unit_keys =
+      page_size >= 16 ? pl.unit_keys_max : (pl.unit_keys_max + page_size - 1) / page_size * 16;
+  if (units <= grid_groups && unit_keys <= short_keys) return lds;
   // More units than resident workgroups, of several heads: the stream's even
   // split wins back its second launch (32/8 heads, 64 sequences of 256 keys,
   // stream / local: 23.1 / 25.7 at head dim 128, 24.7 / 31.8 at 96, 20.1 / 21.7
@@ -560,7 +577,7 @@ int plan_launch(Plan& pl, int32_t batch, int32_t kv_heads, int32_t head_dim,
   }
   const int grid_pairs = lp.groups * (lp.kp.split_waves / 2);
   lp.dim = pl.mf ? head_dim : kernel_dim(head_dim, q8);
-  lp.lds_local = local_lds(pl, batch, kv_heads, lp.dim, q8 ? 1 : 2, lp.kp.gen, fit, page_size,
+  lp.lds_local = local_lds(pl, batch, kv_heads, head_dim, lp.dim, q8 ? 1 : 2, lp.kp.gen, fit, page_size,
                            lp.kp.split_waves, lp.kp.ring, lp.groups);
   // Local mode on the VALU kernels, when a unit per GQA group leaves CUs
   // idle: a unit per query head, as long as the units still fit one

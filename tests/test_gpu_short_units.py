@@ -31,17 +31,20 @@ LINES = [
     (28, 4, 128, 1, 320, "int8", 1, 0), (28, 4, 128, 1, 321, "int8", 0, 2),
     (28, 4, 128, 16, 512, "int8", 1, 0), (28, 4, 128, 16, 513, "int8", 0, 2),
     (8, 4, 256, 1, 256, "int8", 1, 0), (8, 4, 256, 1, 257, "int8", 0, 1),
-    # The generic kernels above head dim 64
-    (32, 8, 96, 1, 448, "int8", 1, 0), (32, 8, 96, 1, 449, "int8", 0, 1),
-    (32, 32, 80, 1, 320, "int8", 1, 0), (32, 32, 80, 1, 321, "int8", 0, 1),
-    (16, 16, 72, 8, 384, "fp16", 1, 0), (16, 16, 72, 8, 385, "fp16", 0, 1),
-    (16, 16, 72, 16, 768, "bf16", 1, 0), (16, 4, 96, 16, 768, "int8", 1, 0),
-    (24, 8, 112, 1, 320, "fp16", 1, 0), (24, 8, 112, 1, 321, "bf16", 0, 1),
-    (24, 8, 112, 16, 128, "fp16", 1, 0), (24, 8, 112, 16, 256, "fp16", 0, 1),
-    (24, 8, 112, 16, 384, "int8", 1, 0), (24, 8, 112, 16, 385, "int8", 0, 1),
-    (8, 8, 160, 1, 192, "bf16", 1, 0), (8, 8, 160, 1, 193, "fp16", 0, 1),
-    (8, 2, 200, 16, 256, "int8", 1, 0), (8, 2, 200, 16, 257, "int8", 0, 1),
-    (8, 2, 200, 64, 64, "fp16", 1, 0), (8, 2, 200, 64, 256, "fp16", 0, 1),
+    # The generic kernels above head dim 64: a workgroup per head (without a GPU,
+    # as here, 256 of them are taken to be resident), a unit's heads together
+    (32, 8, 96, 1, 530, "int8", 1, 0), (32, 8, 96, 1, 531, "int8", 0, 1),
+    (32, 32, 80, 1, 350, "int8", 1, 0), (32, 32, 80, 1, 351, "int8", 0, 1),
+    (16, 16, 72, 1, 391, "fp16", 1, 0), (16, 16, 72, 1, 392, "fp16", 0, 1),
+    (16, 16, 72, 8, 512, "fp16", 1, 0), (16, 16, 72, 8, 513, "fp16", 0, 1),
+    (16, 16, 72, 16, 768, "bf16", 1, 0), (16, 4, 96, 16, 640, "int8", 1, 0),
+    (24, 8, 112, 1, 366, "fp16", 1, 0), (24, 8, 112, 1, 367, "bf16", 0, 1),
+    (64, 8, 112, 1, 566, "fp16", 1, 0), (64, 8, 112, 1, 567, "bf16", 0, 1),
+    (24, 8, 112, 16, 512, "fp16", 1, 0), (24, 8, 112, 16, 513, "int8", 0, 1),
+    (24, 8, 112, 24, 768, "int8", 1, 0),
+    (8, 8, 160, 1, 190, "bf16", 1, 0), (8, 8, 160, 1, 191, "fp16", 0, 1),
+    (8, 2, 200, 16, 280, "int8", 1, 0), (8, 2, 200, 16, 281, "int8", 0, 1),
+    (8, 2, 200, 64, 256, "fp16", 1, 0), (8, 2, 200, 64, 257, "fp16", 0, 1),
     (8, 8, 48, 16, 768, "int8", 1, 0),
 ]
 
@@ -66,6 +69,11 @@ def test_rules_over_wider_tables(hq, hkv, d, batch, longest, kind, local, merge)
         assert choice(hq, hkv, d, batch, longest, kind, width=200)[0] == 1
         assert choice(hq, hkv, d, batch, longest, kind, page=64, width=64)[0] == 1
         assert choice(hq, hkv, d, batch, 4096, kind, width=256, window=longest)[0] == 1
+
+
+def test_rules_with_small_pages():
+    assert choice(28, 4, 128, 17, 1016, "bf16", page=16, width=64, window=512)[0] == 1
+    assert choice(28, 4, 128, 17, 1016, "bf16", page=8, width=127, window=512)[0] == 0
 
 
 def arena(gpu, gen, kind, layout, pages, hkv, d):
