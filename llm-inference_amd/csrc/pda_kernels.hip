@@ -409,7 +409,7 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int head_dim, int dim,
   //    / 198 210 225 249 283; 8 bits: 365 395 459 520 585 / 364 396 468 550 619 /
   //    175 188 232 290 335 / 173 189 240 291 330; 16 x 1 head 505-768, 24 x past
   //    768 (384 above 128 dims);
-  //  257 to 512 heads, two to a CU: 173-485 / 410-536 at 16 / 8 bits, above 128
+  //  257 to 512 heads, two to a CU: 173-485 / 309-536 at 16 / 8 bits, above 128
   //    dims 108-224 / 146-221;
   //  more, together: 16 x 473-614, 24 x past 768; above 128 dims 272-306, past 384.
   // The lines follow the lower of the crossings that share them (16-bit ones by
