@@ -402,38 +402,66 @@ size_t local_lds(const Plan& pl, int batch, int kv_heads, int head_dim, int dim,
                                               : (many || dim < 128 ? 768 : 640);
   // The generic kernels take a wave two to four times as long per key above 64
   // dims, so their lines lie lower, by how a unit's heads run: a workgroup each
-  // (the stream, whose waves take them together, is the slower the more heads),
-  // two of those to a CU, or together. Where local and stream cross, keys, 8 kv
-  // heads, 1, 2, 3, 4, 5 heads a unit; 72 / 112 / 160 / 200 dims:
-  //  1 x, 16 bits: 409 453 515 576 652 / 303 321 361 410 459 / 199 210 230 261 297
-  //    / 198 210 225 249 283; 8 bits: 365 395 459 520 585 / 364 396 468 550 619 /
-  //    175 188 232 290 335 / 173 189 240 291 330; 16 x 1 head 505-768, 24 x past
-  //    768 (384 above 128 dims);
-  //  257 to 512 heads, two to a CU: 173-485 / 309-536 at 16 / 8 bits, above 128
-  //    dims 108-224 / 146-221;
-  //  more, together: 16 x 473-614, 24 x past 768; above 128 dims 272-306, past 384.
-  // The lines follow the lower of the crossings that share them (16-bit ones by
-  // the row's length: 72 dims cross later than 112).
+  // (one to a CU, or two), or together where those would be more than the
+  // resident ones (512; 256 from five heads a unit on). The stream takes a
+  // unit's heads together: the more heads it has, and the more the call has in
+  // all, the later the two cross. Keys where they do, 8 kv heads; 16 bits at 72
+  // / 112 / 200 dims, then 8 bits at 112 / 200:
+  //  one to a CU: 1 x 1 head a unit 409 / 303 / 198, 364 / 173; 1 x 4 576 / 410 /
+  //    249, 550 / 291; 20 x 1 past 768 / 768 / 374, 743 / below 192; 24 x 1 past
+  //    768 (384 above 128 dims), but 8 bits of 200 307; 10 x 2 past 768 / 351 /
+  //    226, 649 / 218; 14 x 2 past 768 / 596 / 234, past 768 / past 384; 8 x 4
+  //    past 768 / 465 / 290, past 768 / 299;
+  //  two: 34 x 1 439 / 295 / 167, 426 / 165; 48 x 1 700 / 462 / 281, past 768 /
+  //    305; 17 x 2 343 / 148 / 103, 187 / 130; 32 x 2 419 / 272 / 114, 428 / 226;
+  //    16 x 4 480 / 198 / 130, 544 / 154;
+  //  together: 8 x 5 415 / 386 / 209, 309 / 144; 13 x 5 667 / 613 / 280, 584 / 152;
+  //    24 x 3 past 768 / past 768 / past 384 at both; from 257 units on two to a
+  //    CU again: 36 x 2 501 / 330 / 166, 430 / 181; 56 x 2 past 768 (384).
   // us, local / stream: 24/8 heads of 112, 16 x 768 keys 49.4 / 28.5; 8/2 of 200,
-  // 64 x 256 31.6 / 22.2; 64/8 of 112, 1 x 341 16.6 / 23.8.
+  // 64 x 256 31.6 / 22.2; 64/8 of 112, 1 x 341 16.6 / 23.8. (The choice is within
+  // 5% of the faster mode at 94 of 100 of 7300 shapes of 120 heads and more that
+  // were timed in both. Times go in steps, so some shapes miss by up to 1.2; units
+  // of one head, more than the resident workgroups, by up to 1.4: 8/8 of 200, 72
+  // x 64 keys 17.4 / 23.7.)
   if (gen && dim > 64 && !fit) {
     const int64_t uh = pl.unit_heads, single = units * uh;
     const bool wide = dim > 128, bits8 = elem == 1;
-    if (single > grid_groups)
-      short_keys = (wide ? 2 : 4) * units;
-    else if (single > 256)  // CUs
-      short_keys = wide                ? (uh >= 5 && !bits8 ? 224 : bits8 ? 150 : 112)
-                   : bits8             ? (uh >= 5 ? 320 : 400)
-                   : head_dim <= 96    ? 384
-                   : uh >= 5           ? 352
-                   : uh == 2           ? 256
-                                       : 192;
-    else
-      short_keys = std::max<int64_t>(wide    ? (bits8 ? 120 + 40 * uh : 170 + 20 * uh)
-                                     : bits8 ? (single >= 192 ? 640 : 290 + 60 * uh)
-                                             : 540 - 21 * head_dim / 8 + 40 * uh,
-                                     units >= (wide ? 192 : 128) ? 4 * units : 0);
-    short_keys = std::min<int64_t>(short_keys, wide ? 384 : 768);
+    const int64_t top = wide ? 384 : 768;
+    if (single > grid_groups) {  // together
+      short_keys = units >= 400  ? top
+                   : units > 256 ? (!wide ? 10 : bits8 ? 5 : 4) * units / 6
+                   : wide        ? (bits8 ? 3 * units - 40 : 2 * units + 80)
+                                 : (bits8 ? 6 * units - 80 : 150 + 9 * units / 2);
+    } else if (single > 256) {  // CUs
+      if (uh == 1 && single >= 384)
+        short_keys = top;
+      else if (wide)
+        short_keys = uh == 1 ? 170 : !bits8 ? 112 : uh == 2 && single >= 448 ? 224 : 150;
+      else if (bits8 || head_dim <= 80)
+        short_keys = uh == 1 ? 3 * single / 2 : single;
+      else
+        short_keys = uh == 1                                       ? single
+                     : uh <= 3 && single >= (uh == 2 ? 384 : 448) ? 256
+                                                                  : 180;
+    } else if (wide) {
+      // (8 bits: two pages a wave, 256 keys, at most: 32/8 heads of 176, 1 x 272
+      // keys 22.1 / 19.6.)
+      short_keys = bits8 ? std::min<int64_t>(120 + 40 * uh, 256) : 170 + 20 * uh + single / 8;
+      if (uh <= 2 && single >= (uh == 1 ? 160 : 224)) short_keys = top;
+    } else if (bits8) {
+      short_keys = single >= 192 ? top : single >= 160 ? 640 : 290 + 60 * uh;
+    } else {
+      short_keys = 540 - 21 * head_dim / 8 + 40 * uh + (uh >= 8 ? 100 : 0);
+      if ((uh <= 2 && single >= 160) || (uh == 3 && single >= 224))
+        short_keys = std::max<int64_t>(short_keys, (head_dim <= 96 ? 7 : 5) * single / 2);
+      if ((head_dim <= 80 && single >= (uh > 3 ? 192 : 160)) ||
+          (head_dim <= 96 && uh >= 4 && single >= 224))
+        short_keys = top;
+    }
+    if (!wide && single <= 256 && units >= 128)
+      short_keys = std::max<int64_t>(short_keys, 4 * units);
+    short_keys = std::min(short_keys, top);
   }
   // (Pages of fewer than 16 keys cost a wave what 16 do: 28/4 heads of 128, 17
   // sequences, a window of 512 in pages of 8: 21.0 / 18.3.)

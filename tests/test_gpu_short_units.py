@@ -39,12 +39,20 @@ LINES = [
     (16, 16, 72, 8, 512, "fp16", 1, 0), (16, 16, 72, 8, 513, "fp16", 0, 1),
     (16, 16, 72, 16, 768, "bf16", 1, 0), (16, 4, 96, 16, 640, "int8", 1, 0),
     (24, 8, 112, 1, 366, "fp16", 1, 0), (24, 8, 112, 1, 367, "bf16", 0, 1),
-    (64, 8, 112, 1, 566, "fp16", 1, 0), (64, 8, 112, 1, 567, "bf16", 0, 1),
-    (24, 8, 112, 16, 512, "fp16", 1, 0), (24, 8, 112, 16, 513, "int8", 0, 1),
+    (64, 8, 112, 1, 666, "fp16", 1, 0), (64, 8, 112, 1, 667, "bf16", 0, 1),
+    (16, 8, 112, 10, 400, "fp16", 1, 0), (16, 8, 112, 10, 401, "bf16", 0, 1),
+    (16, 8, 72, 10, 768, "bf16", 1, 0), (32, 8, 88, 7, 768, "fp16", 1, 0),
+    (16, 8, 112, 10, 640, "int8", 1, 0), (16, 8, 112, 10, 641, "int8", 0, 1),
+    (32, 8, 112, 8, 768, "int8", 1, 0),
+    (40, 8, 112, 8, 438, "fp16", 1, 0), (40, 8, 112, 8, 439, "bf16", 0, 1),
+    (40, 8, 112, 8, 304, "int8", 1, 0), (40, 8, 112, 8, 305, "int8", 0, 1),
+    (32, 8, 112, 17, 762, "fp16", 1, 0), (32, 8, 112, 17, 763, "bf16", 0, 1),
     (24, 8, 112, 24, 768, "int8", 1, 0),
-    (8, 8, 160, 1, 190, "bf16", 1, 0), (8, 8, 160, 1, 191, "fp16", 0, 1),
-    (8, 2, 200, 16, 280, "int8", 1, 0), (8, 2, 200, 16, 281, "int8", 0, 1),
-    (8, 2, 200, 64, 256, "fp16", 1, 0), (8, 2, 200, 64, 257, "fp16", 0, 1),
+    (8, 8, 160, 1, 191, "bf16", 1, 0), (8, 8, 160, 1, 192, "fp16", 0, 1),
+    (8, 8, 160, 20, 384, "fp16", 1, 0),
+    (8, 2, 200, 16, 256, "int8", 1, 0), (8, 2, 200, 16, 257, "int8", 0, 1),
+    (10, 2, 200, 64, 336, "fp16", 1, 0), (10, 2, 200, 64, 337, "fp16", 0, 1),
+    (40, 8, 200, 8, 152, "int8", 1, 0), (40, 8, 200, 8, 177, "int8", 0, 1),
     (8, 8, 48, 16, 768, "int8", 1, 0),
 ]
 
@@ -71,6 +79,24 @@ def test_rules_over_wider_tables(hq, hkv, d, batch, longest, kind, local, merge)
         assert choice(hq, hkv, d, batch, 4096, kind, width=256, window=longest)[0] == 1
 
 
+# Generic kernels of which two workgroups share a CU: more heads than CUs, a
+# workgroup each.
+TWO_TO_A_CU = [
+    (8, 8, 112, 40, 320, "fp16", 1, 0), (8, 8, 112, 40, 321, "fp16", 0, 1),
+    (8, 8, 112, 48, 768, "bf16", 1, 0), (16, 8, 72, 20, 320, "int8", 1, 0),
+    (16, 8, 72, 20, 321, "fp16", 0, 1), (16, 8, 112, 24, 256, "fp16", 1, 0),
+    (16, 8, 112, 24, 257, "fp16", 0, 1), (24, 8, 112, 13, 180, "bf16", 1, 0),
+    (24, 8, 112, 13, 193, "fp16", 0, 1), (16, 8, 200, 28, 224, "int8", 1, 0),
+    (16, 8, 200, 28, 225, "int8", 0, 1),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,d,batch,longest,kind,local,merge", TWO_TO_A_CU)
+def test_rules_two_to_a_cu(gpu, hq, hkv, d, batch, longest, kind, local, merge):
+    assert choice(hq, hkv, d, batch, longest, kind)[0] == local
+
+
 def test_rules_with_small_pages():
     assert choice(28, 4, 128, 17, 1016, "bf16", page=16, width=64, window=512)[0] == 1
     assert choice(28, 4, 128, 17, 1016, "bf16", page=8, width=127, window=512)[0] == 0
@@ -94,7 +120,7 @@ def arena(gpu, gen, kind, layout, pages, hkv, d):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("hq,hkv,d,batch,longest,kind,local,merge", LINES)
+@pytest.mark.parametrize("hq,hkv,d,batch,longest,kind,local,merge", LINES + TWO_TO_A_CU)
 @pytest.mark.parametrize("window,extra,layout", [(0, 0, "pages"), (40, 0, "rows"),
                                                  (0, 50, "rows"), (40, 50, "pages")])
 def test_values(gpu, hq, hkv, d, batch, longest, kind, local, merge, window, extra, layout):
